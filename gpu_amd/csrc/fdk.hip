@@ -801,7 +801,10 @@ __global__ __launch_bounds__(256) void k_fdk_bp_lds(DGeo<float> d, const float4 
                 const float frb = floorf(fminf(fmaxf(khi + 0.5f, -1.0f), Zf)) + 1.0f;
                 const int ca = (int)floorf(fminf(fmaxf(plo - 0.5f, 0.0f), Rf));
                 const int cb = min(max((int)floorf(fminf(fmaxf(phi + 0.5f, 0.0f), Rf)) + 1, ca + 1), min(d.R - 1, ca + 63));
-                const int ra = max((int)fra, 0);
+                // (a tile past the detector's top edge still gets a window of
+                // two rows: with one, the clamp below would let row ZP-1, which
+                // has no row above it, pass the in-detector test)
+                const int ra = max(min((int)fra, d.ZP - 2), 0);
                 const int rb = min(max((int)frb, ra + 1), min(d.ZP - 1, ra + FROWS - 1));
                 if (lane == 0) {
                     wdim[wave] = make_int4(ra, ca, rb - ra + 1, (fra >= 0.0f && frb <= (float)(d.ZP - 1)) ? 1 : 0);
@@ -921,7 +924,8 @@ static ct_status run_fdk_bp(ct_context *ctx, const ct_geometry &g, const void *f
         return launch_check(ctx, "fdk backprojection");
     }
     if constexpr (std::is_same<T, float>::value && !std::is_same<SP, double>::value) {
-        if (ctx->math == CT_MATH_FAST && (uint64_t)g.ncols * g.nrows * sizeof(SP) < (1ull << 32)) {
+        // (one detector row holds no 2x2 stencil: the general kernel leaves the volume as it is)
+        if (ctx->math == CT_MATH_FAST && d.ZP > 1 && (uint64_t)g.ncols * g.nrows * sizeof(SP) < (1ull << 32)) {
             float4 *vt = (float4 *)slot(ctx, SLOT_FDKV, sizeof(float4) * (size_t)nv, &st);
             if (!vt) return st;
             hipLaunchKernelGGL(k_fdk_views, dim3((nv + 255) / 256), dim3(256), 0, ctx->stream, (const float *)ang, vt,

@@ -509,6 +509,21 @@ MS_FDK_G = Geometry(nx=32, ny=30, nz=24, vx=1.0, ncols=64, nrows=24, du=1.0, nvi
                     nsources=3, src_z0=-8.0, src_dz=8.0)
 
 
+@pytest.mark.parametrize("nrows,dv", [(26, 0.966), (1, 1.0)])
+def test_fdk_backprojection_top_edge(ctx, nrows, dv):
+    """Voxels whose stencil row is the detector's last (there is no row above
+    it) get nothing, also in a tile that lies wholly past that row: slices 32
+    to 47 project to 0.06 .. 12 rows above row 25.  One detector row holds no
+    stencil at all.  Against the FP32 restatement at the 1e-5 bar."""
+    g = Geometry(nx=32, ny=32, nz=48, vx=1.0, ncols=64, nrows=nrows, du=1.0, dv=dv, nviews=9)
+    f = np.random.default_rng(8).standard_normal(g.proj_shape).astype(np.float32)
+    v0 = phantom(g, seed=6, scale=0.2).numpy()
+    ref = orc.fdk_backproject(g, f, v0, prec=32)
+    got = host(ctx.fdk_backproject(g, dev(f), dev(v0)))
+    assert rel(got[32:], ref[32:]) <= 1e-5
+    assert rel(got, ref) <= 1e-5
+
+
 @pytest.mark.parametrize("sources", ["inverse_square", "nearest", "equal"])
 def test_multisource_fdk(ctx, sources):
     """Multi-source FDK (TB/FDK): the backprojection with each source
