@@ -575,6 +575,19 @@ def test_ramp_filter_non_power_of_two(ctx):
     assert rel(got, ref) <= 1e-5
 
 
+@pytest.mark.parametrize("ncols", [1, 3, 129, 255, 257, 513, 720, 1025, 2047])
+def test_ramp_filter_transform_lengths(ctx, ncols):
+    """Row lengths around the transform lengths 2^9..2^12, whose taps' spectrum
+    replaces H of the pad 2 ncols; both windows, an odd number of rows, against
+    the FP64 restatement to 1e-5 (FP32 transforms of up to 4096 points round to
+    a few 1e-7)."""
+    g = Geometry(nx=8, ny=8, nz=8, vx=1.0, ncols=ncols, nrows=3, du=0.9, nviews=3, dso=100.0, dod=-50.0)
+    p = np.random.default_rng(ncols).standard_normal((3, 3, ncols)).astype(np.float32)
+    for window in ("ramp", "hann"):
+        ref = orc.ramp_filter(g, p, window, prec=64)
+        assert rel(host(ctx.ramp_filter(g, dev(p), window=window)), ref) <= 1e-5
+
+
 @pytest.mark.parametrize("ncols", [8, 256, 512, 1024, 2048])
 def test_ramp_filter_power_of_two_pads(ctx, ncols):
     """Pads 2^9..2^12 take the Stockham radix-8 kernel, 16 the radix-2 LDS
