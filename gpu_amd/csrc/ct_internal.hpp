@@ -89,6 +89,15 @@ __device__ __forceinline__ float hsub_sat(float a, float b) {
     asm("v_sub_f32_e64 %0, %1, %2 clamp" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
+// hsub_sat(hmin(a, b), hmax(c, d)) as one block: the compiler pads dependent
+// one-instruction blocks with wait states
+__device__ __forceinline__ float hspan(float a, float b, float c, float d) {
+    float r, t;
+    asm("v_min_f32 %0, %2, %3\n\tv_max_f32 %1, %4, %5\n\tv_sub_f32_e64 %0, %0, %1 clamp"
+        : "=&v"(r), "=&v"(t)
+        : "v"(a), "v"(b), "v"(c), "v"(d));
+    return r;
+}
 __device__ __forceinline__ float hmin3(float a, float b, float c) {
     float r;
     asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));

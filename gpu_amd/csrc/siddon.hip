@@ -1139,37 +1139,40 @@ __global__ __launch_bounds__(256) void k_adjoint(DGeo<T> d, const T *__restrict_
 // row.  So each voxel gathers over the pixels of its detector footprint
 // exactly the numbers the walk scatters, in any order and without atomics.
 //
-// Per-view tables: column  (kx, bx0, ky, by0) (lo_xy, hi_xy, i0x|par, i0y|par)
-//                  row     (kz, bz0, lo_z, hi_z) (i0z|par)
+// Per-view tables: column  (kx, bx0, ky, by0) (lo_xy, hi_xy)
+//                  row     (kz, bz0) (lo_z, hi_z)
 //                  pixel   w = dist*y (0 for a ray the forward zeroes)
-// A parallel axis is flagged by i0 >= 0 (the slab the ray stays in); -1
-// marks a stepping axis.
-struct AdjCol { float4 a; float4 b; };
+// A parallel axis (the ray stays in slab i0) gets planes at alpha
+// (n - i0 - 1/2) ADJ_FAR: voxel i0 holds every alpha and any other none.
+struct AdjCol { float4 a; float2 b; };
+constexpr float ADJ_FAR = 1e25f;   // times 2^31 voxels still finite
 
 __device__ __forceinline__ void axis_bounds(float v, float b, int n, float x1, float x2, float &k, float &b0, float &lo,
-                                            float &hi, int &i0, float iv) {
-    // the reference setup's slab interval along this axis
-    // (V63/kernel_IterativeRecon_universal.cu:77-104)
+                                            float &hi, float iv) {
     const float id = 1.0f / (x2 - x1);
-    const float a0 = (b - x1) * id, a1 = (b + v * (float)n - x1) * id;
-    lo = fminf(a0, a1); hi = fmaxf(a0, a1);
     const bool par = v * 1e-6f > fabsf(x1 - x2);
     const PlaneAxis P = plane_axis(v, iv, b, x1, id, 0, par);
-    k = P.k; b0 = P.b0;
-    i0 = par ? P.i0 : -1;
-    if (!par) {
-        const float g0 = b0, gn = fmaf((float)n, k, b0);
-        lo = hmax(lo, hmin(g0, gn));
-        hi = hmin(hi, hmax(g0, gn));
+    if (par) {
+        // a ray outside the grid's slabs has pixel weight 0
+        k = ADJ_FAR;
+        b0 = -((float)P.i0 + 0.5f) * ADJ_FAR;
+        lo = -__builtin_inff(); hi = __builtin_inff();
+        return;
     }
+    // the reference setup's slab interval along this axis
+    // (V63/kernel_IterativeRecon_universal.cu:77-104)
+    const float a0 = (b - x1) * id, a1 = (b + v * (float)n - x1) * id;
+    k = P.k; b0 = P.b0;
+    const float g0 = b0, gn = fmaf((float)n, k, b0);
+    lo = hmax(fminf(a0, a1), hmin(g0, gn));
+    hi = hmin(fmaxf(a0, a1), hmax(g0, gn));
 }
 
 // tables for images [0, nimg) of views view0 + q (q = img / NS)
 template <typename SP>
 __global__ __launch_bounds__(256) void k_adj_prep(DGeo<float> d, const float *__restrict__ ang, int view0,
                                                   const SP *__restrict__ proj, int nimg, float *__restrict__ pixw,
-                                                  AdjCol *__restrict__ colT, float4 *__restrict__ rowA,
-                                                  int *__restrict__ rowB) {
+                                                  AdjCol *__restrict__ colT, float4 *__restrict__ rowT) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int j = blockIdx.y, img = blockIdx.z;
     if (i >= d.R) return;
@@ -1190,35 +1193,19 @@ __global__ __launch_bounds__(256) void k_adj_prep(DGeo<float> d, const float *__
         const float u = d.ymin + (float)i * d.du;
         const float x1x = d.dod * c - u * s, x1y = d.dod * s + u * c;
         float kx, bx0, lx, hx, ky, by0, ly, hy;
-        int ix0, iy0;
-        axis_bounds(d.vx, d.bx, d.M, x1x, x2x, kx, bx0, lx, hx, ix0, d.ivx);
-        axis_bounds(d.vy, d.by, d.N, x1y, x2y, ky, by0, ly, hy, iy0, d.ivy);
+        axis_bounds(d.vx, d.bx, d.M, x1x, x2x, kx, bx0, lx, hx, d.ivx);
+        axis_bounds(d.vy, d.by, d.N, x1y, x2y, ky, by0, ly, hy, d.ivy);
         AdjCol e;
         e.a = make_float4(kx, bx0, ky, by0);
-        e.b = make_float4(hmax(lx, ly), hmin(hx, hy), __int_as_float(ix0), __int_as_float(iy0));
+        e.b = make_float2(hmax(lx, ly), hmin(hx, hy));
         colT[(int64_t)q * d.R + i] = e;
     }
     if (i == 0) {
         const float x1z = d.zmin + (float)j * d.dv;
         const float x2z = d.tb ? (float)(d.sz0 + (float)src * d.sdz) : d.sz0;
         float kz, bz0, lz, hz;
-        int iz0;
-        axis_bounds(d.vz, d.bz, d.Z, x1z, x2z, kz, bz0, lz, hz, iz0, d.ivz);
-        rowA[(int64_t)img * d.ZP + j] = make_float4(kz, bz0, lz, hz);
-        rowB[(int64_t)img * d.ZP + j] = iz0;
-    }
-}
-
-// slab interval [in, out] of voxel index n along one axis for a ray
-__device__ __forceinline__ void slab(float k, float b0, int i0, int n, float &in, float &out) {
-    if (i0 >= 0) {   // parallel: inside slab i0 for all alpha, else never
-        const bool hit = n == i0;
-        in = hit ? -__builtin_inff() : __builtin_inff();
-        out = hit ? __builtin_inff() : -__builtin_inff();
-    } else {
-        const float a0 = fmaf((float)n, k, b0), a1 = fmaf((float)(n + 1), k, b0);
-        in = hmin(a0, a1);
-        out = hmax(a0, a1);
+        axis_bounds(d.vz, d.bz, d.Z, x1z, x2z, kz, bz0, lz, hz, d.ivz);
+        rowT[(int64_t)img * d.ZP + j] = make_float4(kz, bz0, lz, hz);
     }
 }
 
@@ -1228,25 +1215,34 @@ constexpr int ALP = ALW + 8;    // row pitch (zero columns for the NC overrun)
 constexpr int ALH = 48;         // staged footprint rows (48 sources 3 mm apart need 36)
 constexpr int ANC = 8;          // bounding-box columns per voxel
 
-template <int NC>
-__device__ __forceinline__ float adj_rows(const float *__restrict__ sw, const float4 *__restrict__ sra,
-                                          const int *__restrict__ srb, int z0, int z1, int cbase, int iz,
+// One voxel's sum over the rows [z0, z1] of its footprint: per row the slab
+// interval of voxel n along z (planes n and n + 1), per pixel the overlap with
+// the column's x/y interval.  The grid clip of the reference's setup moves a
+// plane only at the grid's own faces (by rounding), so EDGE, the runs that
+// hold a first or last slice, alone applies it.
+template <int NC, bool EDGE>
+__device__ __forceinline__ float adj_rows(const float *__restrict__ sw, const float2 *__restrict__ srk,
+                                          const float2 *__restrict__ srl, int z0, int z1, int cbase, float n, float n1,
                                           const float *xin, const float *xout) {
     float acc = 0.0f;
-    for (int j = z0; j <= z1; ++j) {
-        const float4 ra = sra[j];
-        const float *prow = sw + j * ALP + cbase;
+    const float *prow = sw + (__umul24((uint32_t)z0, ALP) + cbase);
+    const float2 *lp = srl + z0;
+    for (const float2 *rp = srk + z0, *const re = srk + z1; rp <= re; ++rp, prow += ALP) {
+        const float2 rk = *rp;
         float pw[NC];
 #pragma unroll
         for (int cc = 0; cc < NC; ++cc) pw[cc] = prow[cc];
-        float zi, zo;
-        slab(ra.x, ra.y, srb[j], iz, zi, zo);
-        zi = hmax(zi, ra.z);
-        zo = hmin(zo, ra.w);
+        const float a0 = fmaf(n, rk.x, rk.y), a1 = fmaf(n1, rk.x, rk.y);
+        float zi = fminf(a0, a1), zo = fmaxf(a0, a1);
+        if constexpr (EDGE) {
+            const float2 l = *lp++;
+            zi = hmax(zi, l.x);
+            zo = hmin(zo, l.y);
+        }
 #pragma unroll
         for (int cc = 0; cc < NC; ++cc) {
-            const float seg = hsub_sat(hmin(xout[cc], zo), hmax(xin[cc], zi));   // alpha lengths are below 1
-            acc = fmaf(seg, pw[cc], acc);
+            // alpha lengths are below 1
+            acc = fmaf(hspan(xout[cc], zo, xin[cc], zi), pw[cc], acc);
         }
     }
     return acc;
@@ -1254,21 +1250,39 @@ __device__ __forceinline__ float adj_rows(const float *__restrict__ sw, const fl
 
 // one lane per (x, y) and its AZR z-voxels; a 16x16 (x, y) tile per
 // workgroup; per image the tile's detector footprint of weights is staged in
-// LDS.  Each view's per-voxel sum (FP32, ~10 terms) is added into an FP32
+// LDS.  Each image's per-voxel sum (FP32, ~10 terms) is added into an FP32
 // total with Kahan compensation; the volume is written once.
-template <typename SO>
-__global__ __launch_bounds__(256) void k_adjoint_gather(DGeo<float> d, const float *__restrict__ ang, int view0,
-                                                        int nimg, const float *__restrict__ pixw,
+//
+// Bound by VALU issue: 4 per (voxel, footprint pixel), 9 per row and ~20 per
+// voxel.  The columns' x/y intervals are formed once per view and lane, for
+// as many columns as the wave needs, and shared by the run of 8 slices and by
+// the view's sources; each z face's shadow is evaluated once for the two
+// voxels it bounds.  0.32 ms per view at 512^3 / 1024^2 in batches of 16
+// (0.63 ms when every voxel formed all eight columns' and both faces' terms
+// itself), 48 sources x 2 views of 1024 x 128 on 256^3 2.6 ms (5.8).  Four
+// waves per SIMD: five spill (0.41 ms), and a run of 16 slices is no faster
+// (0.33 ms) and needs a third more staged rows.
+//
+// PART: the grid's z axis also splits the views into parts of vpp, for
+// volumes whose tiles leave the chip idle; part p's sums and their
+// compensations go to part[p V + voxel] and k_adj_fold adds them in FP64.
+// 64^3 from 90 views of 96^2: 730 us on its 128 tiles, 80 us in 1024 parts.
+template <typename SO, bool PART>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_adjoint_gather(DGeo<float> d, const float *__restrict__ ang, int view0,
+                                                        int nv, int vpp, const float *__restrict__ pixw,
                                                         const AdjCol *__restrict__ colT,
-                                                        const float4 *__restrict__ rowA, const int *__restrict__ rowB,
-                                                        SO *__restrict__ vol) {
+                                                        const float4 *__restrict__ rowT, SO *__restrict__ vol,
+                                                        float2 *__restrict__ part) {
     __shared__ float sw[ALH * ALP];
-    __shared__ AdjCol sc[ALP];
-    __shared__ float4 sra[ALH];
-    __shared__ int srb[ALH];
+    __shared__ float4 sca[ALP];
+    __shared__ float2 scb[ALP];
+    __shared__ float2 srk[ALH], srl[ALH];
     const int tid = threadIdx.y * 16 + threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6;
     const int3 tile = xcd_tile();
-    const int ix = tile.x * 16 + threadIdx.x, iy = tile.y * 16 + threadIdx.y, iz0 = tile.z * AZR;
+    const int tz = PART ? (d.Z + AZR - 1) / AZR : 1;
+    const int pt = PART ? tile.z / tz : 0;
+    const int ix = tile.x * 16 + threadIdx.x, iy = tile.y * 16 + threadIdx.y, iz0 = (tile.z - pt * tz) * AZR;
     const int nz = min(AZR, d.Z - iz0);
     const bool active = ix < d.M && iy < d.N;
     float cx = 0, cy = 0;
@@ -1279,38 +1293,23 @@ __global__ __launch_bounds__(256) void k_adjoint_gather(DGeo<float> d, const flo
         cx = d.bx + d.vx * (0.5f + (float)ix);
         cy = d.by + d.vy * (0.5f + (float)iy);
     }
-    const float hvx = 0.5f * d.vx, hvy = 0.5f * d.vy, hvz = 0.5f * d.vz;
+    const float hvx = 0.5f * d.vx, hvy = 0.5f * d.vy;
     const float xl = cx - hvx, xh = cx + hvx, yl = cy - hvy, yh = cy + hvy;
+    const float nx = (float)ix, ny = (float)iy;
     const int tx0 = tile.x * 16, ty0 = tile.y * 16;
     const float TX0 = d.bx + (float)tx0 * d.vx, TX1 = d.bx + (float)min(tx0 + 16, d.M) * d.vx;
     const float TY0 = d.by + (float)ty0 * d.vy, TY1 = d.by + (float)min(ty0 + 16, d.N) * d.vy;
     const float TZ0 = d.bz + (float)iz0 * d.vz, TZ1 = d.bz + (float)(iz0 + nz) * d.vz;
+    const bool edge = iz0 == 0 || iz0 + AZR >= d.Z;
     // per-voxel sums over the images, Kahan-compensated FP32
     float W[AZR], Wc[AZR];
 #pragma unroll
     for (int k = 0; k < AZR; ++k) { W[k] = 0.0f; Wc[k] = 0.0f; }
     const int64_t P = (int64_t)d.R * d.ZP;
-    for (int img = 0; img < nimg; ++img) {
-        const int q = img / d.NS, src = img - q * d.NS;
+    const int q1 = PART ? min(nv, (pt + 1) * vpp) : nv;
+    for (int q = PART ? pt * vpp : 0; q < q1; ++q) {
         const int v = view0 + q;
         const float s = ang[2 * v], c = ang[2 * v + 1];
-        const float szs = d.tb ? (float)(d.sz0 + (float)src * d.sdz) : d.sz0;
-        // this lane's voxel column: corner ratios and detector-column box
-        float rmin = __builtin_inff(), rmax = -__builtin_inff(), minY = __builtin_inff(), maxY = -__builtin_inff();
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-            for (int ii = 0; ii < 2; ++ii) {
-                const float px = ii ? xh : xl, py = jj ? yh : yl;
-                const float t = px * c + py * s;
-                const float sv = -px * s + py * c;
-                const float ratio = (t - d.dod) * frcp(d.dso - t);
-                const float u = fmaf(ratio, sv - d.sy, sv);
-                minY = fminf(minY, u); maxY = fmaxf(maxY, u);
-                rmin = fminf(rmin, ratio); rmax = fmaxf(rmax, ratio);
-            }
-        const int y0r = shadow_lo((minY - d.ymin) * d.idu);
-        const int y1r = shadow_hi((maxY - d.ymin) * d.idu);
         // the tile's footprint
         float Tumin = __builtin_inff(), Tumax = -__builtin_inff(), Trmin = __builtin_inff(), Trmax = -__builtin_inff();
 #pragma unroll
@@ -1328,85 +1327,152 @@ __global__ __launch_bounds__(256) void k_adjoint_gather(DGeo<float> d, const flo
         const int C0 = max((int)floorf(fmaf(Tumin - d.ymin, d.idu, 0.5f)) - 1, 0);
         const int C1 = min(min((int)floorf(fmaf(Tumax - d.ymin, d.idu, 0.5f)) + 1, d.R - 1), C0 + ALW - 1);
         const int ncw = C1 - C0 + 1;
-        const float e0 = TZ0 - szs, e1 = TZ1 - szs;
-        const float Tw0 = fminf(fmaf(Trmin, e0, TZ0), fmaf(Trmax, e0, TZ0));
-        const float Tw1 = fmaxf(fmaf(Trmin, e1, TZ1), fmaf(Trmax, e1, TZ1));
-        const int R0 = max((int)floorf(fmaf(Tw0 - d.zmin, d.idv, 0.5f)) - 1, 0);
-        const int R1 = min(min((int)floorf(fmaf(Tw1 - d.zmin, d.idv, 0.5f)) + 1, d.ZP - 1), R0 + ALH - 1);
-        const int nrow = R1 - R0 + 1;
-        if (ncw <= 0 || nrow <= 0) continue;   // uniform
-        __syncthreads();
-        {
-            const float *g = pixw + (int64_t)img * P;
-            for (int i = tid; i < nrow * ALP; i += 256) {
-                const int r = i / ALP, cl = i - r * ALP;
-                sw[i] = cl < ncw ? g[(int64_t)(R0 + r) * d.R + C0 + cl] : 0.0f;
+        if (ncw <= 0) continue;   // uniform
+        // this lane's voxel column: corner ratios and detector-column box
+        float rmin = __builtin_inff(), rmax = -__builtin_inff(), minY = __builtin_inff(), maxY = -__builtin_inff();
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+            for (int ii = 0; ii < 2; ++ii) {
+                const float px = ii ? xh : xl, py = jj ? yh : yl;
+                const float t = px * c + py * s;
+                const float sv = -px * s + py * c;
+                const float ratio = (t - d.dod) * frcp(d.dso - t);
+                const float u = fmaf(ratio, sv - d.sy, sv);
+                minY = fminf(minY, u); maxY = fmaxf(maxY, u);
+                rmin = fminf(rmin, ratio); rmax = fmaxf(rmax, ratio);
             }
-            if (tid < ALP) {
-                AdjCol e;
-                if (tid < ncw) e = colT[(int64_t)q * d.R + C0 + tid];
-                else { e.a = make_float4(0, 0, 0, 0); e.b = make_float4(0, 0, 0, 0); }
-                sc[tid] = e;
-            }
-            if (tid < nrow) {
-                sra[tid] = rowA[(int64_t)img * d.ZP + R0 + tid];
-                srb[tid] = rowB[(int64_t)img * d.ZP + R0 + tid];
-            }
-        }
-        __syncthreads();
-        if (!active) continue;
-        if ((y0r < 0 && y1r < 0) || (y0r > d.R - 1 && y1r > d.R - 1)) continue;
+        const int y0r = shadow_lo((minY - d.ymin) * d.idu);
+        const int y1r = shadow_hi((maxY - d.ymin) * d.idu);
         const int y0 = max(y0r, C0), y1 = min(min(y1r, C1), y0 + ANC - 1);
-        const int ncol = y1 - y0 + 1;
-        if (ncol <= 0) continue;
-        const int cbase = y0 - C0;
-        int NC;
-        if (__builtin_amdgcn_ballot_w64(ncol > 6)) NC = 8;
-        else if (__builtin_amdgcn_ballot_w64(ncol > 4)) NC = 6;
-        else if (__builtin_amdgcn_ballot_w64(ncol > 3)) NC = 4;
-        else NC = 3;
-        // x/y slab interval of this voxel column for each footprint column
+        // (a lane off the volume or the detector has no columns)
+        const int ncol = active ? max(y1 - y0 + 1, 0) : 0;
+        const int cbase = min(max(y0 - C0, 0), ALW - 1);
+        int NC = 0;   // uniform over the wave
+        bool fresh = true;
         float xin[ANC], xout[ANC];
+        for (int src = 0; src < d.NS; ++src) {
+            const int img = q * d.NS + src;
+            const float szs = d.tb ? (float)(d.sz0 + (float)src * d.sdz) : d.sz0;
+            const float e0 = TZ0 - szs, e1 = TZ1 - szs;
+            const float Tw0 = fminf(fmaf(Trmin, e0, TZ0), fmaf(Trmax, e0, TZ0));
+            const float Tw1 = fmaxf(fmaf(Trmin, e1, TZ1), fmaf(Trmax, e1, TZ1));
+            const int R0 = max((int)floorf(fmaf(Tw0 - d.zmin, d.idv, 0.5f)) - 1, 0);
+            const int R1 = min(min((int)floorf(fmaf(Tw1 - d.zmin, d.idv, 0.5f)) + 1, d.ZP - 1), R0 + ALH - 1);
+            const int nrow = R1 - R0 + 1;
+            if (nrow <= 0) continue;   // uniform
+            __syncthreads();   // the previous image's readers are done
+            {
+                // a wave per row, a lane per column; the columns past the
+                // footprint that a voxel's NC columns can reach are zero
+                const float *g = pixw + (int64_t)img * P + (int64_t)R0 * d.R + C0;
+                const bool wide = ncw + 8 > 64;   // uniform
+                for (int r = wave; r < nrow; r += 4) {
+                    sw[r * ALP + lane] = lane < ncw ? g[(int64_t)r * d.R + lane] : 0.0f;
+                    if (wide && lane < ALP - 64)
+                        sw[r * ALP + 64 + lane] = lane + 64 < ncw ? g[(int64_t)r * d.R + 64 + lane] : 0.0f;
+                }
+                if (fresh && tid < ncw) {
+                    const AdjCol e = colT[(int64_t)q * d.R + C0 + tid];
+                    sca[tid] = e.a;
+                    scb[tid] = e.b;
+                }
+                if (tid < nrow) {
+                    const float4 e = rowT[(int64_t)img * d.ZP + R0 + tid];
+                    srk[tid] = make_float2(e.x, e.y);
+                    srl[tid] = make_float2(e.z, e.w);
+                }
+            }
+            __syncthreads();
+            if (fresh) {
+                fresh = false;
+                if (__builtin_amdgcn_ballot_w64(ncol > 6)) NC = 8;
+                else if (__builtin_amdgcn_ballot_w64(ncol > 5)) NC = 6;
+                else if (__builtin_amdgcn_ballot_w64(ncol > 4)) NC = 5;
+                else if (__builtin_amdgcn_ballot_w64(ncol > 3)) NC = 4;
+                else if (__builtin_amdgcn_ballot_w64(ncol > 0)) NC = 3;
+                // x/y slab interval of this voxel column for each footprint
+                // column
 #pragma unroll
-        for (int cc = 0; cc < ANC; ++cc) {
-            const AdjCol e = sc[min(cbase + cc, ALP - 1)];
-            float ai, ao, bi, bo;
-            slab(e.a.x, e.a.y, __float_as_int(e.b.z), ix, ai, ao);
-            slab(e.a.z, e.a.w, __float_as_int(e.b.w), iy, bi, bo);
-            const bool in = cc < ncol;
-            xin[cc] = in ? hmax(hmax(ai, bi), e.b.x) : __builtin_inff();
-            xout[cc] = in ? hmin(hmin(ao, bo), e.b.y) : -__builtin_inff();
-        }
+                for (int cc = 0; cc < ANC; ++cc) {
+                    xin[cc] = __builtin_inff();
+                    xout[cc] = -__builtin_inff();
+                    if (cc >= NC) continue;
+                    const int ci = min(cbase + cc, ncw - 1);
+                    const float4 a = sca[ci];
+                    const float2 b = scb[ci];
+                    const float ax0 = fmaf(nx, a.x, a.y), ax1 = fmaf(nx + 1.0f, a.x, a.y);
+                    const float ay0 = fmaf(ny, a.z, a.w), ay1 = fmaf(ny + 1.0f, a.z, a.w);
+                    if (cc < ncol) {
+                        xin[cc] = hmax(hmax(hmin(ax0, ax1), hmin(ay0, ay1)), b.x);
+                        xout[cc] = hmin(hmin(hmax(ax0, ax1), hmax(ay0, ay1)), b.y);
+                    }
+                }
+            }
+            if (NC == 0) continue;   // uniform over the wave
+            // The faces' shadow rows, counted from the staged window's first
+            // row, with shadow_lo / shadow_hi's margins folded into the
+            // offset: w = z + r (z - z_source) is monotone in the corner
+            // ratio r, so the extreme ratios give its extremes.
+            const float zrow = -d.zmin * d.idv - (float)R0;
+            const float zrow_lo = zrow - 0.01f, zrow_hi = zrow + 0.01f;
+            auto voxels = [&](auto ncc, auto edgec) {
+                constexpr int N = decltype(ncc)::value;
+                constexpr bool E = decltype(edgec)::value;
+                float zk = (float)iz0;
+                asm volatile("" : "+v"(zk));   // the faces are formed here, not kept over the images
+                float zf = fmaf(zk, d.vz, d.bz);
+                float wl = fminf(fmaf(rmin, zf - szs, zf), fmaf(rmax, zf - szs, zf));
 #pragma unroll
-        for (int k = 0; k < AZR; ++k) {
-            if (k >= nz) break;
-            const int iz = iz0 + k;
-            const float cz = !d.tb ? d.bz + d.vz * 0.5f + (float)iz * d.vz : d.bz + d.vz * (0.5f + (float)iz);
-            const float zl = cz - hvz, zh = cz + hvz;
-            const float el = zl - szs, eh = zh - szs;
-            const float wl = fmaf(el >= 0.0f ? rmin : rmax, el, zl);
-            const float wh = fmaf(eh >= 0.0f ? rmax : rmin, eh, zh);
-            int z0 = shadow_lo((wl - d.zmin) * d.idv);
-            int z1 = shadow_hi((wh - d.zmin) * d.idv);
-            if ((z0 < 0 && z1 < 0) || (z0 > d.ZP - 1 && z1 > d.ZP - 1)) continue;
-            z0 = max(z0, R0) - R0;
-            z1 = min(z1, R1) - R0;
-            float a;
-            if (NC == 8) a = adj_rows<8>(sw, sra, srb, z0, z1, cbase, iz, xin, xout);
-            else if (NC == 6) a = adj_rows<6>(sw, sra, srb, z0, z1, cbase, iz, xin, xout);
-            else if (NC == 4) a = adj_rows<4>(sw, sra, srb, z0, z1, cbase, iz, xin, xout);
-            else a = adj_rows<3>(sw, sra, srb, z0, z1, cbase, iz, xin, xout);
-            const float y = a - Wc[k], t = W[k] + y;
-            Wc[k] = (t - W[k]) - y;
-            W[k] = t;
+                for (int k = 0; k < AZR; ++k) {
+                    const float n = zk;
+                    zk += 1.0f;
+                    zf = fmaf(zk, d.vz, d.bz);
+                    const float e = zf - szs;
+                    const float wa = fmaf(rmin, e, zf), wb = fmaf(rmax, e, zf);
+                    const int z0 = max((int)ceilf(fmaf(wl, d.idv, zrow_lo)), 0);
+                    // (slices past the volume have no rows)
+                    const int z1 = min((int)floorf(fmaf(fmaxf(wa, wb), d.idv, zrow_hi)), k < nz ? nrow - 1 : -1);
+                    wl = fminf(wa, wb);
+                    const float a = adj_rows<N, E>(sw, srk, srl, z0, z1, cbase, n, zk, xin, xout);
+                    const float y = a - Wc[k], t = W[k] + y;
+                    Wc[k] = (t - W[k]) - y;
+                    W[k] = t;
+                }
+            };
+            auto by_edge = [&](auto ncc) {
+                if (edge) voxels(ncc, std::true_type());
+                else voxels(ncc, std::false_type());
+            };
+            if (NC == 3) by_edge(std::integral_constant<int, 3>());
+            else if (NC == 4) by_edge(std::integral_constant<int, 4>());
+            else if (NC == 5) by_edge(std::integral_constant<int, 5>());
+            else if (NC == 6) by_edge(std::integral_constant<int, 6>());
+            else by_edge(std::integral_constant<int, 8>());
         }
     }
     if (!active) return;
 #pragma unroll
     for (int k = 0; k < AZR; ++k) {
         if (k >= nz) break;
-        St<SO>::st(vol, ((int64_t)(iz0 + k) * d.N + iy) * d.M + ix, W[k] - Wc[k]);
+        const int64_t idx = ((int64_t)(iz0 + k) * d.N + iy) * d.M + ix;
+        if constexpr (PART) part[(int64_t)pt * ((int64_t)d.M * d.N * d.Z) + idx] = make_float2(W[k], Wc[k]);
+        else St<SO>::st(vol, idx, W[k] - Wc[k]);
     }
+}
+
+// the parts' sums, in part order, in FP64
+template <typename SO>
+__global__ __launch_bounds__(256) void k_adj_fold(const float2 *__restrict__ part, int parts, int64_t V,
+                                                  SO *__restrict__ vol) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= V) return;
+    double a = 0.0;
+    for (int p = 0; p < parts; ++p) {
+        const float2 w = part[(int64_t)p * V + i];
+        a += (double)w.x - (double)w.y;
+    }
+    St<SO>::st(vol, i, (float)a);
 }
 
 // Host bound for k_adjoint_gather: every tile footprint fits ALW x ALH and
@@ -1825,12 +1891,30 @@ static ct_status run_adjoint(ct_context *ctx, const ct_geometry &g, const void *
     return launch_check(ctx, "adjoint");
 }
 
+// Parts the gather's views are split into: enough workgroups for four per CU
+// (what the kernel's registers admit) where the tiles alone give fewer.
+static int adj_parts(const DGeo<float> &d, int nv) {
+    const int64_t tiles = (int64_t)((d.M + 15) / 16) * ((d.N + 15) / 16) * ((d.Z + AZR - 1) / AZR);
+    if (tiles >= 512 || nv < 2) return 1;
+    const int64_t want = std::min<int64_t>((1024 + tiles - 1) / tiles, nv);
+    const int64_t vpp = (nv + want - 1) / want;
+    return (int)((nv + vpp - 1) / vpp);
+}
+
 template <typename SO>
-static void launch_gather(ct_context *ctx, const DGeo<float> &d, const float *ang, int view0, int nimg,
-                          const float *pixw, const AdjCol *colT, const float4 *rowA, const int *rowB, void *vol) {
-    dim3 grid((d.M + 15) / 16, (d.N + 15) / 16, (d.Z + AZR - 1) / AZR);
-    hipLaunchKernelGGL((k_adjoint_gather<SO>), grid, dim3(16, 16, 1), 0, ctx->stream, d, ang, view0, nimg, pixw, colT,
-                       rowA, rowB, (SO *)vol);
+static void launch_gather(ct_context *ctx, const DGeo<float> &d, const float *ang, int view0, int nv, int parts,
+                          const float *pixw, const AdjCol *colT, const float4 *rowT, void *vol, float2 *part) {
+    dim3 grid((d.M + 15) / 16, (d.N + 15) / 16, (d.Z + AZR - 1) / AZR * parts);
+    if (parts == 1) {
+        hipLaunchKernelGGL((k_adjoint_gather<SO, false>), grid, dim3(16, 16, 1), 0, ctx->stream, d, ang, view0, nv, nv,
+                           pixw, colT, rowT, (SO *)vol, part);
+        return;
+    }
+    hipLaunchKernelGGL((k_adjoint_gather<SO, true>), grid, dim3(16, 16, 1), 0, ctx->stream, d, ang, view0, nv,
+                       (nv + parts - 1) / parts, pixw, colT, rowT, (SO *)vol, part);
+    const int64_t V = (int64_t)d.M * d.N * d.Z;
+    hipLaunchKernelGGL((k_adj_fold<SO>), dim3((unsigned)((V + 255) / 256)), dim3(256), 0, ctx->stream,
+                       (const float2 *)part, parts, V, (SO *)vol);
 }
 
 static ct_status run_adjoint_gather(ct_context *ctx, const ct_geometry &g, const DGeo<float> &d, const void *proj,
@@ -1840,27 +1924,29 @@ static ct_status run_adjoint_gather(ct_context *ctx, const ct_geometry &g, const
     if (!ang) return st;
     const int nimg = nv * d.NS;
     const size_t P = (size_t)d.R * d.ZP;
+    const int parts = adj_parts(d, nv);
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t pw_b = up(sizeof(float) * P * nimg), col_b = up(sizeof(AdjCol) * (size_t)d.R * nv);
-    const size_t ra_b = up(sizeof(float4) * (size_t)d.ZP * nimg), rb_b = up(sizeof(int) * (size_t)d.ZP * nimg);
-    char *tab = (char *)slot(ctx, SLOT_TMP_VOL, pw_b + col_b + ra_b + rb_b, &st);
+    const size_t row_b = up(sizeof(float4) * (size_t)d.ZP * nimg);
+    const size_t part_b = parts > 1 ? sizeof(float2) * (size_t)d.M * d.N * d.Z * parts : 0;
+    char *tab = (char *)slot(ctx, SLOT_TMP_VOL, pw_b + col_b + row_b + part_b, &st);
     if (!tab) return st;
     float *pixw = (float *)tab;
     AdjCol *colT = (AdjCol *)(tab + pw_b);
-    float4 *rowA = (float4 *)(tab + pw_b + col_b);
-    int *rowB = (int *)(tab + pw_b + col_b + ra_b);
+    float4 *rowT = (float4 *)(tab + pw_b + col_b);
+    float2 *part = (float2 *)(tab + pw_b + col_b + row_b);
     ProfScope ps(ctx, CT_K_ADJOINT);
     dim3 pg((d.R + 255) / 256, d.ZP, nimg);
     switch (pdt) {
-    case CT_F32: hipLaunchKernelGGL((k_adj_prep<float>), pg, dim3(256), 0, ctx->stream, d, ang, view0, (const float *)proj, nimg, pixw, colT, rowA, rowB); break;
-    case CT_F16: hipLaunchKernelGGL((k_adj_prep<__half>), pg, dim3(256), 0, ctx->stream, d, ang, view0, (const __half *)proj, nimg, pixw, colT, rowA, rowB); break;
-    case CT_BF16: hipLaunchKernelGGL((k_adj_prep<__hip_bfloat16>), pg, dim3(256), 0, ctx->stream, d, ang, view0, (const __hip_bfloat16 *)proj, nimg, pixw, colT, rowA, rowB); break;
+    case CT_F32: hipLaunchKernelGGL((k_adj_prep<float>), pg, dim3(256), 0, ctx->stream, d, ang, view0, (const float *)proj, nimg, pixw, colT, rowT); break;
+    case CT_F16: hipLaunchKernelGGL((k_adj_prep<__half>), pg, dim3(256), 0, ctx->stream, d, ang, view0, (const __half *)proj, nimg, pixw, colT, rowT); break;
+    case CT_BF16: hipLaunchKernelGGL((k_adj_prep<__hip_bfloat16>), pg, dim3(256), 0, ctx->stream, d, ang, view0, (const __hip_bfloat16 *)proj, nimg, pixw, colT, rowT); break;
     default: return fail(ctx, CT_ERR_DTYPE, "unsupported projection dtype");
     }
     switch (vdt) {
-    case CT_F32: launch_gather<float>(ctx, d, ang, view0, nimg, pixw, colT, rowA, rowB, vol); break;
-    case CT_F16: launch_gather<__half>(ctx, d, ang, view0, nimg, pixw, colT, rowA, rowB, vol); break;
-    case CT_BF16: launch_gather<__hip_bfloat16>(ctx, d, ang, view0, nimg, pixw, colT, rowA, rowB, vol); break;
+    case CT_F32: launch_gather<float>(ctx, d, ang, view0, nv, parts, pixw, colT, rowT, vol, part); break;
+    case CT_F16: launch_gather<__half>(ctx, d, ang, view0, nv, parts, pixw, colT, rowT, vol, part); break;
+    case CT_BF16: launch_gather<__hip_bfloat16>(ctx, d, ang, view0, nv, parts, pixw, colT, rowT, vol, part); break;
     default: return fail(ctx, CT_ERR_DTYPE, "unsupported volume dtype");
     }
     return launch_check(ctx, "adjoint");

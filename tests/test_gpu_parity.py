@@ -291,6 +291,23 @@ def test_adjoint_matches_oracle(ctx, name):
     assert rel(got32, ref32) <= 1e-5
 
 
+@pytest.mark.parametrize("nz,nviews,kw", [(9, 1, {}), (9, 2, {}), (17, 67, {}), (7, 5, dict(nsources=3, src_z0=-4.0,
+                                                                                            src_dz=4.0))])
+def test_adjoint_view_parts(ctx, nz, nviews, kw):
+    """The gather adjoint with its views split over workgroups (few tiles):
+    one view, uneven parts, part runs of slices, several sources, and a level
+    row and a central column that run through voxel centres (parallel axes).
+    A 1 mm voxel spans 7.4e-3 of a ray's alpha, whose two crossings round to
+    6e-8 each: 1.6e-5 per segment at most, so 2e-5.  Against the FP32 oracle:
+    rays along the volume's edges are empty in the reference's FP32 set-up and
+    not in FP64."""
+    g = small_geom(nx=25, ny=21, nz=nz, ncols=41, nrows=29, nviews=nviews, **kw)
+    y = np.random.default_rng(nviews).standard_normal(g.proj_shape)
+    ref = orc.adjoint(g, y, prec=32)
+    got = host(ctx.adjoint(g, dev(y)))
+    assert rel(got, ref) <= 2e-5
+
+
 def test_adjoint_multisource_full_size(ctx):
     """The multi-source autograd geometry itself (48 sources 3 mm apart, 1024 x
     128 detector, 256^3 at 0.75 mm): the sources' spread needs 36 footprint
