@@ -638,16 +638,21 @@ __global__ __launch_bounds__(256) void k_project_zq(DGeo<float> d, const float *
 // a zero-length segment), and the sums keep its FP32 batches with a
 // Kahan-compensated FP32 total.  Per segment ~14 VALU (staging included), one
 // LDS pair read and no per-lane gather, against ~25 VALU and one scattered
-// gather per step of the per-ray walk.  Ray-sum batches use it for views
-// whose rays run along x (see col_walk_view); the SART sweep for every view,
-// on a transposed copy of its volume for views whose rays run along y.
-constexpr int COL_ROWS = 256;   // rays per workgroup: rows of one column
+// gather per step of the per-ray walk.  Views whose rays run along y walk a
+// transposed copy of the volume (see col_walk_view).
+// Whether the rays of a view at angle cosine c run along x rather than y (to
+// within ~41 degrees of it).
+__host__ __device__ __forceinline__ bool col_along_x(float c) { return fabsf(c) >= 0.75f; }
+
+// RW, the rays per workgroup (rows of one column): 256, or 128 where that
+// leaves fewer lanes without a row, or where 256 rows span too tall a window
+// (col_plan).
 constexpr int COL_B = 16;       // list padding: a multiple of every staged batch (col_batch)
-constexpr int COL_NQ = 48;      // largest staged window, in z-quads
-// LDS elements per staged window: COL_NQ quads and one quad of padding, so
+template <int RW> constexpr int col_nq() { return RW == 256 ? 48 : 32; }   // largest staged window, in z-quads
+// LDS elements per staged window: col_nq quads and one quad of padding, so
 // that the windows of a batch's segments start on different banks (the
 // staging writes of eight segments' same quad are then conflict-free)
-constexpr int COL_W = 4 * COL_NQ + 4;
+template <int RW> constexpr int col_w() { return 4 * col_nq<RW>() + 4; }
 // List segments per staged batch: 16 (one barrier per 16 segments, and a
 // staging load's eight-lane groups cover 16 segments), or 8 for BF16
 // volumes, whose FP32 windows at 16 would leave four workgroups per CU
@@ -655,7 +660,7 @@ constexpr int COL_W = 4 * COL_NQ + 4;
 // ms and FP16 0.286 -> 0.261 ms from 8 to 16; BF16 0.263 ms at either).
 template <typename SV> constexpr int col_batch() { return std::is_same<SV, __hip_bfloat16>::value ? 8 : 16; }
 // staged quads per thread and batch
-template <typename SV> constexpr int col_sp() { return (col_batch<SV>() * COL_NQ + COL_ROWS - 1) / COL_ROWS; }
+template <typename SV, int RW> constexpr int col_sp() { return (col_batch<SV>() * col_nq<RW>() + RW - 1) / RW; }
 
 // LDS: two staging buffers of col_batch windows in a static array (fixed
 // address and stride, so every staged read has a constant offset; FP32
@@ -669,7 +674,7 @@ template <typename SV> constexpr int col_sp() { return (col_batch<SV>() * COL_NQ
 static inline size_t col_list_entries(int M, int N) { return (size_t)((M + N + COL_B + 3) & ~3); }
 static inline size_t col_dyn_bytes(int M, int N) { return 12 * col_list_entries(M, N); }
 static inline size_t col_lds_bytes(int M, int N) {
-    return sizeof(float) * 2 * COL_B * COL_W + col_dyn_bytes(M, N);
+    return sizeof(float) * 2 * COL_B * col_w<256>() + col_dyn_bytes(M, N);
 }
 
 // Element type of the staged windows: FP16 volumes stage their halves as
@@ -677,19 +682,20 @@ static inline size_t col_lds_bytes(int M, int N) {
 template <typename SV> struct StageOf { using type = float; };
 template <> struct StageOf<__half> { using type = _Float16; };
 
-// TR: the volume is in the transposed z-quad layout [z/4][x][y][z%4], for
-// views whose rays run along y (the staged quads of consecutive segments then
-// share cache lines, as they do along x in the plain z-quad layout).
-template <typename SV, typename SO, typename SM, int CMD, bool TR = false>
-__global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const float *__restrict__ ang,
-                                                          const SV *__restrict__ fq, SO *__restrict__ out,
-                                                          const SM *__restrict__ meas, int first, int stride,
-                                                          int mv0, int z0, int NQ) {
+// fq is the volume in the z-quad layout and ft in its lateral transpose
+// [z/4][x][y][z%4]; a view reads the one along whose fast axis its rays run
+// (col_walk_view: the staged quads of consecutive segments then share cache
+// lines), so one launch takes views of both directions.
+template <typename SV, typename SO, typename SM, int CMD, int RW>
+__global__ __launch_bounds__(RW) void k_project_col(DGeo<float> d, const float *__restrict__ ang,
+                                                          const SV *__restrict__ fq, const SV *__restrict__ ft,
+                                                          SO *__restrict__ out, const SM *__restrict__ meas, int first,
+                                                          int stride, int mv0, int z0, int NQ) {
     using SE = typename StageOf<SV>::type;
     constexpr int SB = (int)sizeof(SE);                // staged bytes per voxel
     constexpr int QSH = SB == 4 ? 4 : 3;               // log2 of the staged bytes per quad
-    constexpr int CB = col_batch<SV>(), SP = col_sp<SV>();
-    __shared__ __align__(16) SE stg[2 * CB * COL_W];
+    constexpr int CB = col_batch<SV>(), SP = col_sp<SV, RW>(), CW = col_w<RW>();
+    __shared__ __align__(16) SE stg[2 * CB * CW];
     extern __shared__ __align__(16) unsigned char col_smem[];
     const int LE = (d.M + d.N + COL_B + 3) & ~3;   // col_list_entries
     float *const la = reinterpret_cast<float *>(col_smem);             // alpha
@@ -698,12 +704,13 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
     constexpr int ES = (int)sizeof(SV);
     const int tid = (int)threadIdx.x;
     const int3 t = xcd_tile();
-    const int col = t.x, row0 = t.y * COL_ROWS, row = row0 + tid;
-    const int rowL = min(row0 + COL_ROWS, d.ZP) - 1;
+    const int col = t.x, row0 = t.y * RW, row = row0 + tid;
+    const int rowL = min(row0 + RW, d.ZP) - 1;
     const int img = t.z + z0;
     const int q = img / d.NS, src = img - q * d.NS;
     const int v = first + q * stride;
     const float s = ang[2 * v], c = ang[2 * v + 1];
+    const bool tr = !col_along_x(c);
     const unsigned M = d.M, MN = (unsigned)d.M * (unsigned)d.N;
     const int ZQ4 = (d.Z + 3) >> 2;                        // quads per (x, y)
     const unsigned QS = MN * 4u * (unsigned)ES;            // bytes between z-quad planes
@@ -747,10 +754,9 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
         const float fsx = (float)sgx, fsy = (float)sgy;
         auto XA = [&](int i) { return fmaf(fmaf((float)i, fsx, px0), X.k, X.b0); };
         auto YA = [&](int j) { return fmaf(fmaf((float)j, fsy, py0), Y.k, Y.b0); };
-        auto OFF = [&](int i, int j) {
-            if constexpr (TR) return (unsigned)(((vi0 + i * sgx) * d.N + (vj0 + j * sgy)) * 4 * ES);
-            else return (unsigned)(((vj0 + j * sgy) * (int)M + (vi0 + i * sgx)) * 4 * ES);
-        };
+        const int ox = (tr ? d.N : 1) * 4 * ES, oy = (tr ? 1 : (int)M) * 4 * ES;
+        const int ox1 = sgx * ox, oy1 = sgy * oy, o0 = vi0 * ox + vj0 * oy;
+        auto OFF = [&](int i, int j) { return (unsigned)(o0 + i * ox1 + j * oy1); };
         // first staged quad of a segment [ap, a]: the z voxel range of the
         // workgroup's first and last rows at both ends, one voxel of margin
         auto QLO = [&](float ap, float a) {
@@ -760,7 +766,7 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
             return vlo >> 2;   // floor division by 4 (arithmetic shift)
         };
         // merge path: thread t writes entries [t C, t C + C); ties take x first
-        const int C = (KP + COL_ROWS - 1) / COL_ROWS;
+        const int C = (KP + RW - 1) / RW;
         const int e0 = tid * C;
         if (e0 < KP) {
             const int ee = min(e0, K);
@@ -811,15 +817,15 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
         // alpha per unit of zeta (0 for a level ray, which never changes slab)
         icz = fabsf(cz) > 1e-30f ? 1.0f / fabsf(cz) : 0.0f;
     }
-    // CMD 0 (ray sums of the autograd pair): the per-ray walk's own segments,
-    // so that the matched adjoint stays its exact transpose.  The lane clips
+    // CMD 0 and 2 (ray sums of the autograd pair, and the objective's residual
+    // of the same sums): the per-ray walk's own segments, so that the matched adjoint stays its exact transpose.  The lane clips
     // the list to its [alpha_min, alpha_max] and tracks its next z-plane
     // crossing fma(nfz, kz, bz0); zrb is its slab relative to kb, times SB.
     float lo = 0.0f, hi = 0.0f, az = __builtin_inff(), nfz = 0.0f, kz = 0.0f, bz0 = __builtin_inff(), sgzf = 0.0f;
     int zrb = 0, dzb = 0;
     if (!cmiss && row < d.ZP && fw.init(d, s, c, col, row, src)) {
         len = fw.len; dist = fw.dist;
-        if constexpr (CMD == 0) {
+        if constexpr (CMD != 1) {
             lo = fw.ac; hi = fw.amax;
             az = fw.az; nfz = fw.nfz; kz = fw.kz; bz0 = fw.bz0; sgzf = fw.sgzf;
             zrb = ((int)nfz - (sgzf > 0.0f ? 1 : 0)) * SB - kbb;
@@ -828,10 +834,10 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
     }
     const bool up = cz >= 0.0f;
     const unsigned nbytes = MN * (unsigned)ZQ4 * 4u * (unsigned)ES;
-    const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(fq, nbytes);
+    const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(tr ? ft : fq, nbytes);
     // this thread's staged quads (the same in every batch): segment k of the
     // batch and quad qi of its window (sk = -1: none), and where they go
-    const int nst = CB * NQ;   // quads staged per batch (at most SP * COL_ROWS)
+    const int nst = CB * NQ;   // quads staged per batch (at most SP * RW)
     // Segment-fastest: lanes 8q .. 8q + 7 load quad q of the batch's eight
     // segments.  Consecutive segments are mostly neighbours along the
     // layout's fast axis, whose quads share a 128-byte line, so a wave's load
@@ -840,10 +846,10 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
     int sk[SP], sq[SP], so[SP];
 #pragma unroll
     for (int p = 0; p < SP; ++p) {
-        const int sidx = tid + p * COL_ROWS;
+        const int sidx = tid + p * RW;
         sk[p] = sidx < nst ? sidx % CB : -1;
         sq[p] = sidx / CB;
-        so[p] = (sidx % CB) * COL_W + 4 * sq[p];
+        so[p] = (sidx % CB) * CW + 4 * sq[p];
     }
     // a quad outside the volume reads as zeros: its index is clamped to -1 or
     // ZQ4, whose offsets lie past the buffer's end (the volume is under 2 GiB)
@@ -875,7 +881,7 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
 #pragma unroll
         for (int p = 0; p < SP; ++p) {
             if (sk[p] < 0) continue;
-            SE *const dst = stg + (buf * CB * COL_W + so[p]);
+            SE *const dst = stg + (buf * CB * CW + so[p]);
             if constexpr (std::is_same<SV, __hip_bfloat16>::value) {
                 const uint2 r = sreg[p];
                 *reinterpret_cast<float4 *>(dst) = make_float4(__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u),
@@ -897,7 +903,7 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
     // CMD 1 (SART corrections): a segment [as, ae] of the column's list lies
     // in one x/y voxel; this ray
     // enters it in slab k = floor(zeta(as)) and, as |dzeta| < 1 per segment
-    // (col_walk_nq), crosses at most one z plane in it.  The crossing part,
+    // (col_plan), crosses at most one z plane in it.  The crossing part,
     // in zeta units clamp(zeta(ae) - (k + 1), 0, 1) for a rising ray or
     // clamp(k - zeta(ae), 0, 1) for a falling one, times alpha per unit of
     // zeta, belongs to the next slab and the rest of the segment to slab k;
@@ -917,7 +923,7 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
             const float wy = (ae - as) - wx;
             const int klo = (int)kf - (UP ? 0 : 1);
             const unsigned a = min((unsigned)(klo * SB + ew[k]), wmax2);
-            const SE *pr = reinterpret_cast<const SE *>(sb + k * COL_W * SB + a);
+            const SE *pr = reinterpret_cast<const SE *>(sb + k * CW * SB + a);
             const float f0 = (float)pr[0], f1 = (float)pr[1];
             ps = fmaf(UP ? wy : wx, f0, ps);
             ps = fmaf(UP ? wx : wy, f1, ps);
@@ -944,8 +950,8 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
             nfz += cr ? sgzf : 0.0f;
             az = fmaf(nfz, kz, bz0);
             const unsigned r1 = min((unsigned)(zrb + ew[k]), wmax);
-            ps = fmaf(d0, (float)*reinterpret_cast<const SE *>(sb + k * COL_W * SB + r0), ps);
-            ps = fmaf(d1, (float)*reinterpret_cast<const SE *>(sb + k * COL_W * SB + r1), ps);
+            ps = fmaf(d0, (float)*reinterpret_cast<const SE *>(sb + k * CW * SB + r0), ps);
+            ps = fmaf(d1, (float)*reinterpret_cast<const SE *>(sb + k * CW * SB + r1), ps);
             asx = ae;
         }
         return ps;
@@ -956,7 +962,7 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
         constexpr int BUF = decltype(bufc)::value;
         __syncthreads();   // batch b staged; batch b - 1's readers are done with the other buffer
         if (b + 1 < nb) issue(b + 1);
-        const char *sb = reinterpret_cast<const char *>(stg + BUF * CB * COL_W);
+        const char *sb = reinterpret_cast<const char *>(stg + BUF * CB * CW);
         float ea[CB];
         int ew[CB];
 #pragma unroll
@@ -969,7 +975,7 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
         }
         // rising and falling rays (all but one wave per column are uniform)
         float ps;
-        if constexpr (CMD == 0) ps = segs_exact(sb, ea, ew);
+        if constexpr (CMD != 1) ps = segs_exact(sb, ea, ew);
         else ps = up ? segs(std::true_type(), sb, ea, ew) : segs(std::false_type(), sb, ea, ew);
         const float yk = ps - comp;
         const float tk = sum + yk;
@@ -981,20 +987,37 @@ __global__ __launch_bounds__(COL_ROWS) void k_project_col(DGeo<float> d, const f
         batch(std::integral_constant<int, 0>(), b);
         if (b + 1 < nb) batch(std::integral_constant<int, 1>(), b + 1);
     }
-    if (row >= d.ZP) return;
     const int64_t P = (int64_t)d.R * d.ZP;
     const int64_t pix = (int64_t)row * d.R + col;
-    float r = 0.0f;
-    if (!(len < d.vz * 1e-6f)) {
-        const float ax = (sum - comp) * dist;
-        if constexpr (CMD == 0) r = ax;
-        else r = ((float)ldf(meas, ((int64_t)(v - mv0) * d.NS + src) * P + pix) - ax) / len;
+    const float ax = len < d.vz * 1e-6f ? 0.0f : (sum - comp) * dist;
+    if constexpr (CMD == 2) {
+        // FP64 sum of the workgroup's squared residuals, one slot per workgroup
+        __shared__ double wsum[RW / 64];
+        double e2 = 0.0;
+        if (row < d.ZP) {
+            const double e = (double)ax - (double)ldf(meas, ((int64_t)(v - mv0) * d.NS + src) * P + pix);
+            e2 = e * e;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) e2 += __shfl_down(e2, o, 64);
+        if ((tid & 63) == 0) wsum[tid >> 6] = e2;
+        __syncthreads();
+        if (tid == 0)
+            out[((int64_t)img * gridDim.y + t.y) * gridDim.x + t.x] =
+                RW == 256 ? (wsum[0] + wsum[1]) + (wsum[RW / 64 - 2] + wsum[RW / 64 - 1]) : wsum[0] + wsum[1];
+        return;
     }
-    St<SO>::st(out, (int64_t)img * P + pix, r);
+    if (row >= d.ZP) return;
+    float r = ax;
+    if constexpr (CMD == 1)
+        r = len < d.vz * 1e-6f ? 0.0f : ((float)ldf(meas, ((int64_t)(v - mv0) * d.NS + src) * P + pix) - ax) / len;
+    if constexpr (CMD != 2) St<SO>::st(out, (int64_t)img * P + pix, r);
 }
 
 // Data fidelity sum (Ax - b)^2 fused into the ray traversal: Ax never goes to
-// memory.  Each 256-ray block writes one FP64 partial (wave64 shuffles, then
+// memory.  Geometries that admit the column walk take it (CMD 2 of
+// k_project_col); this per-ray form serves the others, exact mode and FP64.
+// Each 256-ray block writes one FP64 partial (wave64 shuffles, then
 // LDS across the 4 waves); the partials are folded in fixed order afterwards.
 // (L2_norm_gpu + the objective's Forward_3D_ray_driven_siddon,
 // V63/host_tool_functions.cu:28-58 and V63/main_recon.cu:401-407.)
@@ -1028,59 +1051,6 @@ __global__ __launch_bounds__(256) void k_residual(DGeo<T> d, const T *__restrict
     if (threadIdx.x == 0)
         part[((int64_t)z0 * gridDim.y + blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] =
             (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
-}
-
-template <typename T, typename SV, typename SM>
-static ct_status run_residual(ct_context *ctx, const ct_geometry &g, const void *vol, const void *meas, double *out) {
-    ct_status st;
-    const T *ang = (const T *)angle_table(ctx, g, sizeof(T) == 8, false, &st);
-    if (!ang) return st;
-    DGeo<T> d = derive<T>(g);
-    const int nimg = g.nviews * d.NS;
-    const int gx = (d.R + 15) / 16, gy = (d.ZP + 15) / 16;
-    const int64_t nblk = (int64_t)gx * gy * nimg;
-    double *part = (double *)slot(ctx, SLOT_TMP_PROJ2, sizeof(double) * nblk, &st);
-    if (!part) return st;
-    const bool comp = std::is_same<T, float>::value && ctx->math == CT_MATH_FAST;
-    {
-        ProfScope ps(ctx, CT_K_FORWARD);
-        for (int z0 = 0; z0 < nimg; z0 += 65535) {
-            const int nz = nimg - z0 < 65535 ? nimg - z0 : 65535;
-            dim3 grid(gx, gy, nz);
-            if (comp)
-                hipLaunchKernelGGL((k_residual<T, SV, SM, true>), grid, dim3(256), 0, ctx->stream, d, ang,
-                                   (const SV *)vol, (const SM *)meas, 0, z0, part);
-            else
-                hipLaunchKernelGGL((k_residual<T, SV, SM, false>), grid, dim3(256), 0, ctx->stream, d, ang,
-                                   (const SV *)vol, (const SM *)meas, 0, z0, part);
-        }
-    }
-    st = launch_check(ctx, "residual");
-    if (st != CT_OK) return st;
-    return reduce_dot(ctx, part, nullptr, nblk, CT_F64, 2, out);
-}
-
-template <typename T, typename SV>
-static ct_status residual_meas(ct_context *ctx, const ct_geometry &g, const void *vol, const void *meas, ct_dtype mdt,
-                               double *out) {
-    switch (mdt) {
-    case CT_F32: return run_residual<T, SV, float>(ctx, g, vol, meas, out);
-    case CT_F16: return run_residual<T, SV, __half>(ctx, g, vol, meas, out);
-    case CT_BF16: return run_residual<T, SV, __hip_bfloat16>(ctx, g, vol, meas, out);
-    case CT_F64: return run_residual<T, SV, double>(ctx, g, vol, meas, out);
-    }
-    return fail(ctx, CT_ERR_DTYPE, "residual: bad measurement dtype");
-}
-
-ct_status launch_residual(ct_context *ctx, const ct_geometry &g, const void *vol, ct_dtype vdt, const void *meas,
-                          ct_dtype mdt, double *out) {
-    switch (vdt) {
-    case CT_F32: return residual_meas<float, float>(ctx, g, vol, meas, mdt, out);
-    case CT_F16: return residual_meas<float, __half>(ctx, g, vol, meas, mdt, out);
-    case CT_BF16: return residual_meas<float, __hip_bfloat16>(ctx, g, vol, meas, mdt, out);
-    case CT_F64: return residual_meas<double, double>(ctx, g, vol, meas, mdt, out);
-    }
-    return fail(ctx, CT_ERR_DTYPE, "residual: bad volume dtype");
 }
 
 template <typename A> __device__ __forceinline__ void atomic_add(A *p, A v);
@@ -1501,8 +1471,8 @@ static bool adj_gather_fits(const DGeo<float> &d) {
     return cols(DT) + 4.0 <= ALW && rows(DT, AZR * vz) + 4.0 <= ALH && cols(DV) + 2.0 <= ANC;
 }
 
-// Host conditions of k_project_col; returns the staged window NQ (quads per
-// segment) or 0.  The list and two staging buffers fit the workgroup's LDS,
+// Host conditions of k_project_col; gives the rows per workgroup and the
+// staged window NQ (quads per segment).  The list and two staging buffers fit the workgroup's LDS,
 // the z-quad volume is under 2 GiB, and no list segment holds two z
 // crossings: along every ray |dz|/vz < max(|dx|/vx, |dy|/vy), checked with
 // |dz| at its largest (rows against the farthest source height) and the
@@ -1515,17 +1485,20 @@ static bool adj_gather_fits(const DGeo<float> &d) {
 // fan and parallel rays keep their row height.  One voxel of the segment's
 // own z travel, one of rounding margin on each side and the quad alignment
 // are added.
-static int col_walk_nq(const DGeo<float> &d) {
-    if ((uint64_t)d.M * d.N * (uint64_t)((d.Z + 3) & ~3) * 4 >= (1ull << 31)) return 0;
-    if ((d.ZP + COL_ROWS - 1) / COL_ROWS > 65535) return 0;
-    double dzmax = 0.0;
+// Of the two workgroup sizes the one with fewer lanes past the last row, and
+// 256 rows at a tie: at 512^3 / 1024^2, where both fill, a view takes 0.34 ms
+// with 256 and 0.36 ms with 128 (FP32; each workgroup makes its own list).
+// With 128 an FP16 correction of 1000 x 830 on 500 x 468 x 391 takes 0.26 ms
+// against 0.28, the gradient of 90 views of 96^2 on 64^3 163 us against 217,
+// and the 128^3 / 256^2 sweep in subsets of 20, whose 256 rows overrun the
+// window, 2.48 ms against 2.70 with the per-ray walk.
+struct ColPlan { int rows, nq; };   // nq 0: the walk is not admitted
+static int col_quads(const DGeo<float> &d, int rw, int max_nq) {
+    if ((d.ZP + rw - 1) / rw > 65535) return 0;
     const double inplane = std::fabs((double)d.dso - (double)d.dod);
-    const int rows = std::min(COL_ROWS, d.ZP) - 1;
+    const int rows = std::min(rw, d.ZP) - 1;
     double span;
     if (d.style == CT_CONE) {
-        const double s0 = d.sz0, s1 = d.tb ? d.sz0 + (double)(d.NS - 1) * d.sdz : d.sz0;
-        dzmax = std::max(std::max(std::fabs(d.zmin - s0), std::fabs(d.zmax - s0)),
-                         std::max(std::fabs(d.zmin - s1), std::fabs(d.zmax - s1)));
         const double X0 = d.bx, X1 = d.bx + (double)d.M * d.vx, Y0 = d.by, Y1 = d.by + (double)d.N * d.vy;
         const double rxy = std::sqrt(std::max(X0 * X0, X1 * X1) + std::max(Y0 * Y0, Y1 * Y1));
         const double rho = (rxy + std::hypot((double)d.dso, (double)d.sy)) / inplane;
@@ -1533,61 +1506,201 @@ static int col_walk_nq(const DGeo<float> &d) {
     } else {
         span = rows * (double)d.dv / (double)d.vz;
     }
-    const double vxy = std::max((double)d.vx, (double)d.vy);
-    if (!(dzmax / (double)d.vz < 0.9 * inplane / (std::sqrt(2.0) * vxy))) return 0;
     const double nq = std::ceil((span + 8.0) / 4.0);
-    if (!(nq >= 1.0) || nq > COL_NQ) return 0;
+    return nq >= 1.0 && nq <= max_nq ? (int)nq : 0;
+}
+static ColPlan col_plan(const DGeo<float> &d) {
+    const ColPlan none = {0, 0};
+    if ((uint64_t)d.M * d.N * (uint64_t)((d.Z + 3) & ~3) * 4 >= (1ull << 31)) return none;
+    double dzmax = 0.0;
+    const double inplane = std::fabs((double)d.dso - (double)d.dod);
+    if (d.style == CT_CONE) {
+        const double s0 = d.sz0, s1 = d.tb ? d.sz0 + (double)(d.NS - 1) * d.sdz : d.sz0;
+        dzmax = std::max(std::max(std::fabs(d.zmin - s0), std::fabs(d.zmax - s0)),
+                         std::max(std::fabs(d.zmin - s1), std::fabs(d.zmax - s1)));
+    }
+    const double vxy = std::max((double)d.vx, (double)d.vy);
+    if (!(dzmax / (double)d.vz < 0.9 * inplane / (std::sqrt(2.0) * vxy))) return none;
     // (the padding of col_dyn_lds keeps a workgroup under 33 KiB)
-    if (col_lds_bytes(d.M, d.N) > 65536) return 0;
-    return (int)nq;
+    if (col_lds_bytes(d.M, d.N) > 65536) return none;
+    const int n256 = col_quads(d, 256, col_nq<256>()), n128 = col_quads(d, 128, col_nq<128>());
+    const int pad256 = (d.ZP + 255) / 256 * 256, pad128 = (d.ZP + 127) / 128 * 128;
+    if (n128 > 0 && (n256 == 0 || pad128 < pad256)) return {128, n128};
+    return {n256 > 0 ? 256 : 0, n256};
 }
 
-// Dynamic LDS of a launch: the list, padded so that a workgroup holds at
-// least col_lds_floor bytes in all, which caps the workgroups per CU.
+// Dynamic LDS of a launch: the list, padded so that a workgroup of 256 holds
+// at least col_lds_floor bytes in all, which caps the workgroups per CU.
 // Measured per view at 512^3 / 1024^2 (a one-view launch is 4096
 // workgroups): FP32 volumes 0.457 ms at four per CU against 0.464 at five and
 // 0.485 at six; FP16 0.331 ms at four against 0.376 at seven; BF16 (windows
 // staged as FP32) 0.378 ms at six against 0.436 at four.
-template <typename SV> constexpr size_t col_lds_floor() {
-    return std::is_same<SV, __hip_bfloat16>::value ? 0 : 32 * 1024 + 512;   // > 160 KiB / 5
+template <typename SV, int RW> constexpr size_t col_lds_floor() {
+    return std::is_same<SV, __hip_bfloat16>::value || RW != 256 ? 0 : 32 * 1024 + 512;   // > 160 KiB / 5
 }
-template <typename SV> static size_t col_dyn_lds(int M, int N) {
-    const size_t stat = sizeof(typename StageOf<SV>::type) * 2 * col_batch<SV>() * COL_W + 16;
-    const size_t want = col_lds_floor<SV>();
+template <typename SV, int RW> static size_t col_dyn_lds(int M, int N) {
+    const size_t stat = sizeof(typename StageOf<SV>::type) * 2 * col_batch<SV>() * col_w<RW>() + 16;
+    const size_t want = col_lds_floor<SV, RW>();
     const size_t list = col_dyn_bytes(M, N);
     return stat + list >= want ? list : want - stat;
 }
-template <typename SV, typename SO, typename SM, int CMD, bool TR = false>
-static void launch_col(ct_context *ctx, const DGeo<float> &d, int nq, const float *ang, const void *volq, void *out,
-                       const void *meas, int first, int stride, int mv0, int nimg) {
+template <typename SV, typename SO, typename SM, int CMD, int RW>
+static void launch_col_rw(ct_context *ctx, const DGeo<float> &d, int nq, const float *ang, const void *const vols[2],
+                          void *out, const void *meas, int first, int stride, int mv0, int nimg) {
     for (int z0 = 0; z0 < nimg; z0 += 65535) {
         const int nz = nimg - z0 < 65535 ? nimg - z0 : 65535;
-        dim3 grid(d.R, (d.ZP + COL_ROWS - 1) / COL_ROWS, nz);
-        hipLaunchKernelGGL((k_project_col<SV, SO, SM, CMD, TR>), grid, dim3(COL_ROWS), col_dyn_lds<SV>(d.M, d.N),
-                           ctx->stream, d, ang, (const SV *)volq, (SO *)out, (const SM *)meas, first, stride, mv0,
-                           z0, nq);
+        dim3 grid(d.R, (d.ZP + RW - 1) / RW, nz);
+        hipLaunchKernelGGL((k_project_col<SV, SO, SM, CMD, RW>), grid, dim3(RW), (col_dyn_lds<SV, RW>(d.M, d.N)),
+                           ctx->stream, d, ang, (const SV *)vols[0], (const SV *)vols[1], (SO *)out, (const SM *)meas,
+                           first, stride, mv0, z0, nq);
     }
 }
 
 // The column walk stages, per segment, one z-quad of each (x, y) on the
-// column's path; a 128-byte line holds eight x-neighbours, so paths that run
-// along x use whole lines and paths along y one quad per line.  Measured at
-// 512^3 / 1024^2 per view: 0.39 vs 0.46 ms (per-ray walk) along x, even near
-// 40 degrees, 0.67 vs 0.44 ms along y.  Views whose central ray is within
-// ~41 degrees of the x axis (|cos| >= 0.75) take the column walk; by_run
-// splits a launch's views into runs of one choice.
-static bool col_walk_view(const ct_geometry &g, int v) { return std::fabs(view_cos(g, v)) >= 0.75f; }
-template <typename F> static void by_run(const ct_geometry &g, bool allow, int first, int stride, int nv, F &&launch) {
-    int q0 = 0;
-    bool cur = allow && nv > 0 && col_walk_view(g, first);
-    for (int q = 1; q < nv; ++q) {
-        const bool cw = allow && col_walk_view(g, first + q * stride);
-        if (cw != cur) { launch(q0, q - q0, cur); q0 = q; cur = cw; }
+// column's path; a 128-byte line holds eight neighbours along the layout's
+// fast axis, so paths that run along it use whole lines and paths across it
+// one quad per line.  Measured at 512^3 / 1024^2 per view: 0.39 ms along the
+// fast axis, even near 40 degrees, 0.67 ms across it.  Views whose central
+// ray is within ~41 degrees of the x axis (|cos| >= 0.75) walk the z-quad
+// copy, the others its lateral transpose.
+static bool col_walk_view(const ct_geometry &g, int v) { return col_along_x(view_cos(g, v)); }
+
+// Per-ray walk on the z-quad layout (k_project_zq): one walk per ray for ray
+// sums, each ray split in two for corrections.
+template <typename SV, typename SO, typename SM, int CMD>
+static void launch_zq(ct_context *ctx, const DGeo<float> &d, const float *ang, const void *volq, SO *out,
+                      const void *meas, int first, int stride, int nimg, int mv0) {
+    constexpr int S = CMD == 1 ? CORR_SPLIT : 1;
+    constexpr int tw = S <= 2 ? 16 : 8, th = S == 1 ? 16 : 8;
+    for (int z0 = 0; z0 < nimg; z0 += 65535) {
+        const int nz = nimg - z0 < 65535 ? nimg - z0 : 65535;
+        dim3 grid((d.R + tw - 1) / tw, (d.ZP + th - 1) / th, nz);
+        hipLaunchKernelGGL((k_project_zq<SV, SO, SM, CMD, S>), grid, dim3(256), 0, ctx->stream, d, ang,
+                           (const SV *)volq, out, (const SM *)meas, first, stride, mv0, z0);
     }
-    if (nv > 0) launch(q0, nv - q0, cur);
+}
+
+// Walks the views first, first + stride, ... of a z-quad volume by column.
+// volq is in the plain layout or, with `tr`, the transposed one (each in its
+// own slot of the context).  Views that run the other way need the other copy
+// (0.17 ms at 512^3 in FP32), which pays from the first view on FP32 volumes
+// (0.59 -> 0.39 ms per view there), but for 16-bit ones, whose per-ray walk
+// is nearly as fast (358 x 342 x 339 / 718 x 707 in FP16: 0.154 -> 0.149 ms
+// per view, the copy 0.036 ms), only from eight images on; fewer take the
+// per-ray walk on volq.
+template <typename SV, typename SO, typename SM, int CMD>
+static ct_status launch_col(ct_context *ctx, const ct_geometry &g, const DGeo<float> &d, ColPlan cp, const float *ang,
+                            const void *volq, bool tr, void *out, const void *meas, int first, int stride, int nv,
+                            int mv0) {
+    const void *vols[2] = {volq, volq};
+    auto walk = [&](int q0, int n, void *o) {
+        if (cp.rows == 256) launch_col_rw<SV, SO, SM, CMD, 256>(ctx, d, cp.nq, ang, vols, o, meas, first + q0 * stride, stride, mv0, n * d.NS);
+        else launch_col_rw<SV, SO, SM, CMD, 128>(ctx, d, cp.nq, ang, vols, o, meas, first + q0 * stride, stride, mv0, n * d.NS);
+    };
+    int others = 0;
+    for (int q = 0; q < nv; ++q) others += col_walk_view(g, first + q * stride) == tr;
+    if constexpr (CMD != 2 && sizeof(SV) == 2) {
+        if (others > 0 && others * d.NS < 8 && !tr) {
+            const int64_t P = (int64_t)d.R * d.ZP * d.NS;
+            for (int q0 = 0, q1; q0 < nv; q0 = q1) {
+                const bool w = col_walk_view(g, first + q0 * stride);
+                for (q1 = q0 + 1; q1 < nv && col_walk_view(g, first + q1 * stride) == w; ++q1) {}
+                SO *o = (SO *)out + q0 * P;
+                if (w) walk(q0, q1 - q0, o);
+                else launch_zq<SV, SO, SM, CMD>(ctx, d, ang, volq, o, meas, first + q0 * stride, stride, (q1 - q0) * d.NS, mv0);
+            }
+            return CT_OK;
+        }
+    }
+    if (others > 0) {
+        ct_status st;
+        const uint64_t bytes = (uint64_t)d.M * d.N * (uint64_t)((d.Z + 3) & ~3) * sizeof(SV);
+        void *t = slot(ctx, tr ? SLOT_ZQVOL : SLOT_ZQVOL_T, bytes, &st);
+        if (!t) return st;
+        st = launch_zq_transpose(ctx, volq, dtype_of<SV>(), t, d.M, d.N, d.Z, !tr);
+        if (st != CT_OK) return st;
+        vols[!tr] = t;
+    }
+    walk(0, nv, out);
+    return CT_OK;
 }
 
 // ---------------------------------------------------------------- launchers
+template <typename T, typename SV, typename SM>
+static ct_status run_residual(ct_context *ctx, const ct_geometry &g, const void *vol, const void *meas, double *out) {
+    ct_status st;
+    const T *ang = (const T *)angle_table(ctx, g, sizeof(T) == 8, false, &st);
+    if (!ang) return st;
+    DGeo<T> d = derive<T>(g);
+    const int nimg = g.nviews * d.NS;
+    const bool comp = std::is_same<T, float>::value && ctx->math == CT_MATH_FAST;
+    if constexpr (std::is_same<T, float>::value) {
+        // the batched ray sums' column walk, on the same conditions
+        const uint64_t qbytes = (uint64_t)d.M * d.N * (uint64_t)((d.Z + 3) & ~3) * sizeof(SV);
+        const ColPlan cp = comp && nimg >= 4 && qbytes < (1ull << 32) ? col_plan(d) : ColPlan{0, 0};
+        if (cp.nq > 0) {
+            const int64_t per = (int64_t)d.R * ((d.ZP + cp.rows - 1) / cp.rows);   // workgroups per image
+            double *part = (double *)slot(ctx, SLOT_TMP_PROJ2, sizeof(double) * per * nimg, &st);
+            if (!part) return st;
+            void *volq = slot(ctx, SLOT_ZQVOL, qbytes, &st);
+            if (!volq) return st;
+            {
+                ProfScope ps(ctx, CT_K_FORWARD);
+                st = launch_zq_pack(ctx, vol, dtype_of<SV>(), volq, d.M, d.N, d.Z);
+                if (st != CT_OK) return st;
+                st = launch_col<SV, double, SM, 2>(ctx, g, d, cp, ang, volq, false, part, meas, 0, 1, g.nviews, 0);
+                if (st != CT_OK) return st;
+            }
+            st = launch_check(ctx, "residual");
+            if (st != CT_OK) return st;
+            return reduce_dot(ctx, part, nullptr, per * nimg, CT_F64, 2, out);
+        }
+    }
+    const int gx = (d.R + 15) / 16, gy = (d.ZP + 15) / 16;
+    const int64_t nblk = (int64_t)gx * gy * nimg;
+    double *part = (double *)slot(ctx, SLOT_TMP_PROJ2, sizeof(double) * nblk, &st);
+    if (!part) return st;
+    {
+        ProfScope ps(ctx, CT_K_FORWARD);
+        for (int z0 = 0; z0 < nimg; z0 += 65535) {
+            const int nz = nimg - z0 < 65535 ? nimg - z0 : 65535;
+            dim3 grid(gx, gy, nz);
+            if (comp)
+                hipLaunchKernelGGL((k_residual<T, SV, SM, true>), grid, dim3(256), 0, ctx->stream, d, ang,
+                                   (const SV *)vol, (const SM *)meas, 0, z0, part);
+            else
+                hipLaunchKernelGGL((k_residual<T, SV, SM, false>), grid, dim3(256), 0, ctx->stream, d, ang,
+                                   (const SV *)vol, (const SM *)meas, 0, z0, part);
+        }
+    }
+    st = launch_check(ctx, "residual");
+    if (st != CT_OK) return st;
+    return reduce_dot(ctx, part, nullptr, nblk, CT_F64, 2, out);
+}
+
+template <typename T, typename SV>
+static ct_status residual_meas(ct_context *ctx, const ct_geometry &g, const void *vol, const void *meas, ct_dtype mdt,
+                               double *out) {
+    switch (mdt) {
+    case CT_F32: return run_residual<T, SV, float>(ctx, g, vol, meas, out);
+    case CT_F16: return run_residual<T, SV, __half>(ctx, g, vol, meas, out);
+    case CT_BF16: return run_residual<T, SV, __hip_bfloat16>(ctx, g, vol, meas, out);
+    case CT_F64: return run_residual<T, SV, double>(ctx, g, vol, meas, out);
+    }
+    return fail(ctx, CT_ERR_DTYPE, "residual: bad measurement dtype");
+}
+
+ct_status launch_residual(ct_context *ctx, const ct_geometry &g, const void *vol, ct_dtype vdt, const void *meas,
+                          ct_dtype mdt, double *out) {
+    switch (vdt) {
+    case CT_F32: return residual_meas<float, float>(ctx, g, vol, meas, mdt, out);
+    case CT_F16: return residual_meas<float, __half>(ctx, g, vol, meas, mdt, out);
+    case CT_BF16: return residual_meas<float, __hip_bfloat16>(ctx, g, vol, meas, mdt, out);
+    case CT_F64: return residual_meas<double, double>(ctx, g, vol, meas, mdt, out);
+    }
+    return fail(ctx, CT_ERR_DTYPE, "residual: bad volume dtype");
+}
+
 template <typename T, typename SV, typename SO, typename SM, int CMD>
 static ct_status run_forward(ct_context *ctx, const ct_geometry &g, const void *vol, void *out, const void *meas,
                              int first, int stride, int nv, int mv0) {
@@ -1612,24 +1725,13 @@ static ct_status run_forward(ct_context *ctx, const ct_geometry &g, const void *
             ProfScope ps(ctx, CT_K_FORWARD);   // the copy is part of the call's cost
             st = launch_zq_pack(ctx, vol, dtype_of<SV>(), volq, d.M, d.N, d.Z);
             if (st != CT_OK) return st;
-            const int nq = col_walk_nq(d);
-            const int64_t P = (int64_t)d.R * d.ZP;
-            by_run(g, nq > 0, first, stride, nv, [&](int q0, int n, bool cw) {
-                SO *o = (SO *)out + (int64_t)q0 * d.NS * P;
-                const int f0 = first + q0 * stride, ni = n * d.NS;
-                if (cw) {
-                    launch_col<SV, SO, SM, CMD>(ctx, d, nq, ang, volq, o, meas, f0, stride, mv0, ni);
-                    return;
-                }
-                constexpr int S = CMD == 1 ? CORR_SPLIT : 1;
-                constexpr int tw = S <= 2 ? 16 : 8, th = S == 1 ? 16 : 8;
-                for (int z0 = 0; z0 < ni; z0 += 65535) {
-                    const int nz = ni - z0 < 65535 ? ni - z0 : 65535;
-                    dim3 grid((d.R + tw - 1) / tw, (d.ZP + th - 1) / th, nz);
-                    hipLaunchKernelGGL((k_project_zq<SV, SO, SM, CMD, S>), grid, dim3(256), 0, ctx->stream, d, ang,
-                                       (const SV *)volq, o, (const SM *)meas, f0, stride, mv0, z0);
-                }
-            });
+            const ColPlan cp = col_plan(d);
+            if (cp.nq > 0) {
+                st = launch_col<SV, SO, SM, CMD>(ctx, g, d, cp, ang, volq, false, out, meas, first, stride, nv, mv0);
+                if (st != CT_OK) return st;
+            } else {
+                launch_zq<SV, SO, SM, CMD>(ctx, d, ang, volq, (SO *)out, meas, first, stride, nimg, mv0);
+            }
             return launch_check(ctx, "forward");
         }
     }
@@ -1663,7 +1765,10 @@ static ct_status fwd_meas(ct_context *ctx, const ct_geometry &g, const void *vol
 template <typename T, typename SV, int CMD>
 static ct_status fwd_out(ct_context *ctx, const ct_geometry &g, const void *vol, void *out, ct_dtype odt,
                          const void *meas, ct_dtype mdt, int first, int stride, int nv, int mv0) {
-    switch (odt) {
+    if constexpr (CMD == 1) {   // corrections are in the arithmetic type
+        if (odt != dtype_of<T>()) return fail(ctx, CT_ERR_DTYPE, "unsupported output dtype");
+        return fwd_meas<T, SV, T, CMD>(ctx, g, vol, out, meas, mdt, first, stride, nv, mv0);
+    } else switch (odt) {
     case CT_F32: return fwd_meas<T, SV, float, CMD>(ctx, g, vol, out, meas, mdt, first, stride, nv, mv0);
     case CT_F16: return fwd_meas<T, SV, __half, CMD>(ctx, g, vol, out, meas, mdt, first, stride, nv, mv0);
     case CT_BF16: return fwd_meas<T, SV, __hip_bfloat16, CMD>(ctx, g, vol, out, meas, mdt, first, stride, nv, mv0);
@@ -1801,30 +1906,16 @@ static ct_status run_correction_zq(ct_context *ctx, const ct_geometry &g, const 
     if (!ang) return st;
     DGeo<float> d = derive<float>(g);
     ProfScope ps(ctx, CT_K_FORWARD);
-    const int nq = col_walk_nq(d);
-    const int64_t P = (int64_t)d.R * d.ZP;
-    if (tr) {
-        // transposed layout (sweep_view_transposed held for the caller's
-        // views): every view takes the column walk
-        if (nq <= 0) return fail(ctx, CT_ERR_INVALID_ARG, "transposed correction without the column walk");
-        launch_col<SV, float, SM, 1, true>(ctx, d, nq, ang, volq, corr, meas, first, stride, 0, nv * d.NS);
-        return launch_check(ctx, "correction");
+    const ColPlan cp = col_plan(d);
+    if (cp.nq > 0) {
+        // (a subset's views may run both ways; the update that follows works
+        // on volq, so the other copy serves this correction alone)
+        st = launch_col<SV, float, SM, 1>(ctx, g, d, cp, ang, volq, tr, corr, meas, first, stride, nv, 0);
+        return st != CT_OK ? st : launch_check(ctx, "correction");
     }
-    by_run(g, nq > 0, first, stride, nv, [&](int q0, int n, bool cw) {
-        float *o = corr + (int64_t)q0 * d.NS * P;
-        const int f0 = first + q0 * stride, ni = n * d.NS;
-        if (cw) {
-            launch_col<SV, float, SM, 1>(ctx, d, nq, ang, volq, o, meas, f0, stride, 0, ni);
-            return;
-        }
-        for (int z0 = 0; z0 < ni; z0 += 65535) {
-            const int nz = ni - z0 < 65535 ? ni - z0 : 65535;
-            constexpr int tw = CORR_SPLIT <= 2 ? 16 : 8, th = CORR_SPLIT == 1 ? 16 : 8;
-            dim3 grid((d.R + tw - 1) / tw, (d.ZP + th - 1) / th, nz);
-            hipLaunchKernelGGL((k_project_zq<SV, float, SM, 1, CORR_SPLIT>), grid, dim3(256), 0, ctx->stream, d, ang,
-                               (const SV *)volq, o, (const SM *)meas, f0, stride, 0, z0);
-        }
-    });
+    // (only with the column walk does the sweep use the transposed layout)
+    if (tr) return fail(ctx, CT_ERR_INVALID_ARG, "transposed correction without the column walk");
+    launch_zq<SV, float, SM, 1>(ctx, d, ang, volq, corr, meas, first, stride, nv * d.NS, 0);
     return launch_check(ctx, "correction");
 }
 
@@ -1857,7 +1948,7 @@ ct_status launch_correction_zq(ct_context *ctx, const ct_geometry &g, const void
 // The sweep walks views whose rays run along y on the transposed z-quad
 // layout, so that every view takes the column walk with line-sharing staging.
 bool sweep_view_transposed(const ct_geometry &g, int v) {
-    return !col_walk_view(g, v) && col_walk_nq(derive<float>(g)) > 0;
+    return !col_walk_view(g, v) && col_plan(derive<float>(g)).nq > 0;
 }
 
 ct_status launch_forward(ct_context *ctx, const ct_geometry &g, const void *vol, ct_dtype vdt, void *out,

@@ -291,6 +291,23 @@ def test_adjoint_matches_oracle(ctx, name):
     assert rel(got32, ref32) <= 1e-5
 
 
+@pytest.mark.parametrize("nrows", [1, 64, 65, 128, 129, 256, 257])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_column_walk_row_blocks(ctx, nrows, dt):
+    """Ray sums and the objective of views of both directions in one launch,
+    with the rows of a column in blocks of 128 or 256 and part blocks, at the
+    1e-5 projection bar against the FP32 oracle on the stored volume."""
+    g = small_geom(nrows=nrows, dv=30.8 / nrows, ncols=21, nviews=11)
+    x = torch.as_tensor(phantom(g, seed=5, scale=0.3)).to("cuda", dt)
+    ref = orc.forward(g, host(x).astype(np.float32), prec=32)
+    assert rel(host(ctx.forward(g, x, out_dtype=torch.float32)), ref) <= 1e-5
+    meas = (0.5 * ref + 0.01).astype(np.float32)
+    data, _, _ = ctx.objective(g, x, dev(meas))
+    want = float(((ref.astype(np.float64) - meas) ** 2).sum())
+    # |Ax - b| <= |Ax| + |b| and b = Ax/2 + 0.01: the 1e-5 of Ax is at most 2e-5 of the residual each way
+    assert abs(data - want) <= 4e-5 * want
+
+
 @pytest.mark.parametrize("nz,nviews,kw", [(9, 1, {}), (9, 2, {}), (17, 67, {}), (7, 5, dict(nsources=3, src_z0=-4.0,
                                                                                             src_dz=4.0))])
 def test_adjoint_view_parts(ctx, nz, nviews, kw):
