@@ -445,163 +445,187 @@ __global__ __launch_bounds__(256) void k_fgp_L(const S *b, const D *r, const D *
     if (Lout) { if constexpr (std::is_same<S, double>::value) Lout[v] = L; else St<S>::st(Lout, v, L); }
 }
 
-// One FGP inner iteration in one pass (L never goes to memory).  The dual
-// fields are double-buffered: the pass reads r, s, t of the previous
-// iteration from one set and writes the next iteration's to the other, so a
-// workgroup can read its neighbours' old values at the tile borders whatever
-// their progress.  A workgroup owns a 128 x 8 (x, y) tile and marches a chunk
-// of z slices: it stages the old r, s, t of the next slice in LDS with a
-// one-voxel border, forms L of that slice on the tile and its right column
-// and bottom row (the neighbours the dual step needs), then updates the
-// current slice.  Per voxel the arithmetic is that of k_fgp_L followed by the
-// dual gradient step, unit-ball projection and momentum of FGP_operator_LT_Pp
-// (V63/kernel_FGP_Denoise_GPUx7.cu:27-88).  HBM traffic ~13.8 words per voxel (13 for b, the old duals, o,
-// p, q read and the new duals, o, p, q written; the rest is the staged
-// border) against 18 for the two-kernel form.
-constexpr int FGX = 128, FGY = 8;            // tile (threads)
-constexpr int FEX = FGX + 2, FEY = FGY + 2;  // staged extent: one voxel of border
-constexpr int FLX = FGX + 1, FLY = FGY + 1;  // L extent: tile + right column + bottom row
-constexpr int FGZ = 64;                      // slices per workgroup
+// A lane's value from the lane below / above it in the wave; lane 0 / lane 63
+// takes `edge`.
+__device__ __forceinline__ float lane_below(float v, float edge) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(edge), __float_as_int(v), 0x138, 0xf, 0xf, false));   // wave_shr:1
+}
+__device__ __forceinline__ float lane_above(float v, float edge) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(edge), __float_as_int(v), 0x130, 0xf, 0xf, false));   // wave_shl:1
+}
+__device__ __forceinline__ double lane_below(double v, double edge) {
+    const double u = __shfl_up(v, 1, 64);
+    return threadIdx.x == 0 ? edge : u;
+}
+__device__ __forceinline__ double lane_above(double v, double edge) {
+    const double u = __shfl_down(v, 1, 64);
+    return threadIdx.x == 63 ? edge : u;
+}
+// lane l's value, uniform
+__device__ __forceinline__ float lane_value(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double lane_value(double v, int l) { return __shfl(v, l, 64); }
 
-template <typename S, typename T, typename D = T>
-__global__ __launch_bounds__(FGX * FGY) void k_fgp_step(const S *__restrict__ b, const D *__restrict__ rA,
-                                                        const D *__restrict__ sA, const D *__restrict__ tA,
-                                                        D *__restrict__ rB, D *__restrict__ sB, D *__restrict__ tB,
-                                                        D *__restrict__ o, D *__restrict__ p, D *__restrict__ q, int M,
-                                                        int N, int Z, T lambda, T g, T a12) {
-    // staged old duals: three slices in flight (written one step ahead of
-    // their first reader, so no barrier guards the write); L: two slices
-    __shared__ T sr[3][FEY * FEX], ss[3][FEY * FEX], stt[3][FEY * FEX];
-    __shared__ T sL[2][FLY * FLX];
-    constexpr int NT = FGX * FGY;
-    const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * FGX + tx;
-    // x/y neighbours on one XCD: their border lines meet in its L2
-    const int3 tile = xcd_tile();
-    const int i0 = tile.x * FGX, j0 = tile.y * FGY;
-    const int k0 = tile.z * FGZ, k1 = min(k0 + FGZ, Z);
-    if (k0 >= k1) return;
-    const int64_t MN = (int64_t)M * N;
-    // this thread's staged and L entries (the same in every slice): offset
-    // in the slice, or -1 outside the volume / past the extent
-    int soff[2], loff[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        const int e = tid + u * NT;
-        soff[u] = -1; loff[u] = -1;
-        if (e < FEX * FEY) {
-            const int ly = e / FEX - 1, lx = e - (ly + 1) * FEX - 1;
-            const int i = i0 + lx, j = j0 + ly;
-            if (i >= 0 && i < M && j >= 0 && j < N) soff[u] = j * M + i;
-        }
-        if (e < FLX * FLY) {
-            const int ly = e / FLX, lx = e - ly * FLX;
-            const int i = i0 + lx, j = j0 + ly;
-            if (i < M && j < N) loff[u] = j * M + i;
-        }
-    }
-    // every load of a slice is issued one step before its use: the staged
-    // duals (extended tile, zero outside the volume), b on the L extent and
-    // the owner's o, p, q; held in their raw storage form until used
+// One FGP inner iteration in one pass: neither L nor the momentum point goes
+// to memory.  The iteration keeps its projected duals P of the last two
+// iterations; the momentum point (r, s, t) = P1 + g (P1 - P0) is formed where
+// it is read, with the operations that FGP_operator_LT_Pp
+// (V63/kernel_FGP_Denoise_GPUx7.cu:27-88) ends on, L from it as k_fgp_L does,
+// then the dual gradient step and the unit-ball projection of
+// FGP_operator_LT_Pp give the next P in a third set, so neighbours read old
+// values whatever their progress.  HBM per voxel: 7 words read (b, two sets)
+// and 3 written, against 13 when the momentum point was kept too.
+//
+// A wave owns 64 x FGR (x, y) columns and marches a chunk of z slices with
+// everything in registers: a lane is one x, its x neighbours are lanes away,
+// its y neighbours its own registers; no LDS, no barriers, and the loads of a
+// slice are issued one step before their use, in raw form.  Rows above (s
+// only) and below (L) are read as well.  The columns beside the 64 come with
+// one more load per array, whose lanes are rows: lanes 1 .. FGR + 1 hold the
+// right column x0 + 64 and form its L, lanes 16 + a the points of x0 + 63
+// next to it and lanes 32 + a those of the left column x0 - 1 (lane 0: s of
+// the row above).
+//
+// FIRST 2: no duals yet (all zero); 1: one set, whose momentum factor is 0.
+// The waves of a workgroup lie side by side in x (2^lx of them, the rest
+// stacked in y), so that it touches whole rows of up to 1 KiB: with the waves
+// stacked in y instead the pass takes 1.25 ms at 512^3 in FP32, side by side
+// 1.04 (4.9 TB/s over its 10 words; a large copy runs at 4.6), against 1.38
+// for the form with LDS staging and the momentum point in memory.  FP16 on 500
+// x 468 x 391: 0.87 -> 0.55 ms.
+constexpr int FGW = 4;                       // waves per workgroup
+
+template <typename S, typename T, typename D, int FIRST, int FGR>
+__global__ __launch_bounds__(64 * FGW) void k_fgp_step(const S *__restrict__ b, const D *__restrict__ rA,
+                                                       const D *__restrict__ sA, const D *__restrict__ tA,
+                                                       const D *__restrict__ rO, const D *__restrict__ sO,
+                                                       const D *__restrict__ tO, D *__restrict__ rN,
+                                                       D *__restrict__ sN, D *__restrict__ tN, int M, int N, int Z,
+                                                       int lx, int zc, T lambda, T g, T a12) {
     using RD = typename RawOf<D>::type;
     using RS = typename RawOf<S>::type;
-    RD gr[2], gs[2], gt[2];
-    RS gb[2];
-    auto fetch_stage = [&](int k) {
+    const int3 tile = xcd_tile();
+    const int lane = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int x0 = ((tile.x << lx) + (wave & ((1 << lx) - 1))) * 64, i = x0 + lane;
+    const int j0 = (tile.y * (FGW >> lx) + (wave >> lx)) * FGR;
+    const int k0 = tile.z * zc, k1 = min(k0 + zc, Z);
+    if (x0 >= M || j0 >= N || k0 >= k1) return;
+    const int64_t MN = (int64_t)M * N;
+    // lanes off the volume read its edge; what they form is never used
+    const unsigned ic = (unsigned)min(i, M - 1);
+    // this lane's element of the side columns: its offset in a slice
+    const int hg = lane >> 4, ha = (lane & 15) - (hg == 0);
+    const unsigned hoff = (unsigned)(min(max(j0 + ha, 0), N - 1) * M + min(max(x0 + (hg == 0 ? 64 : hg == 1 ? 63 : -1), 0), M - 1));
+    const bool hcol = hg == 0 && ha <= FGR;            // the right column, with the row above
+    const bool hr = hg < 3 && ha >= 0 && ha <= FGR;    // the points r beside it
+    RD pr[FGR + 1], ps[FGR + 1], pt[FGR + 1], qr[FGR + 1], qs[FGR + 1], qt[FGR + 1], psa = 0, qsa = 0;
+    RD hpr = 0, hps = 0, hpt = 0, hqr = 0, hqs = 0, hqt = 0;
+    RS pb[FGR + 1], hb = 0;
+    auto row = [&](int k, int j) { return (int64_t)k * MN + (int64_t)min(j, N - 1) * M; };
+    auto fetch = [&](int k) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            gr[u] = 0; gs[u] = 0; gt[u] = 0;
-            if (soff[u] >= 0) {
-                const int64_t v = (int64_t)k * MN + soff[u];
-                gr[u] = ld_raw(rA, v); gs[u] = ld_raw(sA, v); gt[u] = ld_raw(tA, v);
+        for (int a = 0; a <= FGR; ++a) {
+            const int64_t v = row(k, j0 + a);
+            pb[a] = ld_raw(b + v, ic);
+            if constexpr (FIRST < 2) { pr[a] = ld_raw(rA + v, ic); ps[a] = ld_raw(sA + v, ic); pt[a] = ld_raw(tA + v, ic); }
+            if constexpr (FIRST < 1) { qr[a] = ld_raw(rO + v, ic); qs[a] = ld_raw(sO + v, ic); qt[a] = ld_raw(tO + v, ic); }
+        }
+        if (j0 > 0) {
+            const int64_t v = row(k, j0 - 1);
+            if constexpr (FIRST < 2) psa = ld_raw(sA + v, ic);
+            if constexpr (FIRST < 1) qsa = ld_raw(sO + v, ic);
+        }
+        const int64_t v = (int64_t)k * MN;
+        if (hr) {
+            if constexpr (FIRST < 2) hpr = ld_raw(rA + v, hoff);
+            if constexpr (FIRST < 1) hqr = ld_raw(rO + v, hoff);
+        }
+        if (hcol) {
+            hb = ld_raw(b + v, hoff);
+            if constexpr (FIRST < 2) { hps = ld_raw(sA + v, hoff); hpt = ld_raw(tA + v, hoff); }
+            if constexpr (FIRST < 1) { hqs = ld_raw(sO + v, hoff); hqt = ld_raw(tO + v, hoff); }
+        }
+    };
+    // the momentum point from the last two projections
+    auto point = [&](RD p, RD q) {
+        if constexpr (FIRST == 2) return (T)0;
+        const T on = from_raw<T, D>(p);
+        if constexpr (FIRST == 1) return on;
+        return on + g * (on - from_raw<T, D>(q));
+    };
+    // slice k's point and L from the fetched values, with its t and the t of
+    // slice k - 1; hL, ht: L and t of the right column, by row
+    T r[FGR + 1], s[FGR + 1], t[FGR + 1], L[FGR + 1], hL, ht;
+    auto form = [&](T (&rk)[FGR + 1], T (&sk)[FGR + 1], T (&tk)[FGR + 1], const T (&tm)[FGR + 1], T (&Lk)[FGR + 1],
+                    T &hLk, T &htk, T htm) {
+        const T h = point(hpr, hqr), hs = point(hps, hqs);
+        htk = point(hpt, hqt);
+        {
+            const T hm = __shfl(h, lane + 15, 64);   // r at x0 + 63 of this lane's row
+            const T hsm = lane_below(hs, (T)0);
+            const T tl = (h - hm) + (hs - (j0 + ha > 0 ? hsm : (T)0)) + (htk - htm);
+            hLk = from_raw<T, S>(hb) - lambda * tl;
+        }
+        T sm = j0 > 0 ? point(psa, qsa) : (T)0;
+#pragma unroll
+        for (int a = 0; a <= FGR; ++a) {
+            rk[a] = point(pr[a], qr[a]); sk[a] = point(ps[a], qs[a]); tk[a] = point(pt[a], qt[a]);
+            const T left = lane_below(rk[a], lane_value(h, 32 + a));
+            const T rm = i > 0 ? left : (T)0;
+            const T tl = (rk[a] - rm) + (sk[a] - sm) + (tk[a] - tm[a]);
+            Lk[a] = from_raw<T, S>(pb[a]) - lambda * tl;
+            sm = sk[a];
+        }
+    };
+    {
+        T tm[FGR + 1];
+        RD hp = 0, hq = 0;
+#pragma unroll
+        for (int a = 0; a <= FGR; ++a) {
+            tm[a] = (T)0;
+            if (k0 > 0) {
+                const int64_t v = row(k0 - 1, j0 + a);
+                RD p = 0, q = 0;
+                if constexpr (FIRST < 2) p = ld_raw(tA + v, ic);
+                if constexpr (FIRST < 1) q = ld_raw(tO + v, ic);
+                tm[a] = point(p, q);
             }
         }
-    };
-    auto put_stage = [&](int k) {
-        const int bf = k % 3;
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int e = tid + u * NT;
-            if (e < FEX * FEY) {
-                sr[bf][e] = from_raw<T, D>(gr[u]); ss[bf][e] = from_raw<T, D>(gs[u]);
-                stt[bf][e] = from_raw<T, D>(gt[u]);
-            }
+        if (k0 > 0 && hcol) {
+            const int64_t v = (int64_t)(k0 - 1) * MN;
+            if constexpr (FIRST < 2) hp = ld_raw(tA + v, hoff);
+            if constexpr (FIRST < 1) hq = ld_raw(tO + v, hoff);
         }
-    };
-    auto fetch_b = [&](int k) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            gb[u] = 0;
-            if (loff[u] >= 0) gb[u] = ld_raw(b, (int64_t)k * MN + loff[u]);
-        }
-    };
-    // L of slice k on the tile + right column + bottom row (k_fgp_L)
-    auto formL = [&](int k, const RS (&bv)[2]) {
-        const int bf = k % 3, pf = (k + 2) % 3;   // slices k and k - 1
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int e = tid + u * NT;
-            if (e >= FLX * FLY) continue;
-            const int ly = e / FLX, lx = e - ly * FLX;
-            const int i = i0 + lx, j = j0 + ly;
-            T L = 0;
-            if (i < M && j < N) {
-                const int c = (ly + 1) * FEX + (lx + 1);
-                const T rm = i > 0 ? sr[bf][c - 1] : (T)0;
-                const T sm = j > 0 ? ss[bf][c - FEX] : (T)0;
-                const T tm = k > 0 ? stt[pf][c] : (T)0;
-                const T tl = (sr[bf][c] - rm) + (ss[bf][c] - sm) + (stt[bf][c] - tm);
-                L = from_raw<T, S>(bv[u]) - lambda * tl;
-            }
-            sL[k & 1][e] = L;
-        }
-    };
-    const int i = i0 + tx, j = j0 + ty;
-    const bool own = i < M && j < N;
-    RD po = 0, pp = 0, pq = 0;
-    auto fetch_own = [&](int k) {
-        if (own) {
-            const int64_t v = (int64_t)k * MN + (int64_t)j * M + i;
-            po = ld_raw(o, v); pp = ld_raw(p, v); pq = ld_raw(q, v);
-        }
-    };
-    // prologue: slices k0 - 1 and k0 staged, L(k0) formed, slice k0 + 1's
-    // duals, b of k0 + 1 and the owner's o, p, q of k0 in flight
-    if (k0 > 0) { fetch_stage(k0 - 1); put_stage(k0 - 1); }
-    fetch_stage(k0); put_stage(k0);
-    fetch_b(k0);
-    __syncthreads();
-    formL(k0, gb);
-    if (k0 + 1 < Z) { fetch_stage(k0 + 1); fetch_b(k0 + 1); }
-    fetch_own(k0);
+        fetch(k0);
+        form(r, s, t, tm, L, hL, ht, point(hp, hq));
+    }
+    if (k0 + 1 < Z) fetch(k0 + 1);
     for (int k = k0; k < k1; ++k) {
+        T rn[FGR + 1], sn[FGR + 1], tn[FGR + 1], Ln[FGR + 1], hLn, htn;
         const bool nx = k + 1 < Z;
-        if (nx) put_stage(k + 1);
-        const RD co = po, cp = pp, cq = pq;
-        const RS bn[2] = {gb[0], gb[1]};
-        if (k + 2 < Z && k + 1 < k1) { fetch_stage(k + 2); fetch_b(k + 2); }
-        if (k + 1 < k1) fetch_own(k + 1);
-        __syncthreads();   // slice k + 1 staged; L(k) complete
-        if (nx) formL(k + 1, bn);
-        __syncthreads();   // L(k + 1) complete
-        if (!own) continue;
-        // dual step, projection and momentum (FGP_operator_LT_Pp)
-        const int64_t v = (int64_t)k * MN + (int64_t)j * M + i;
-        const int c = (ty + 1) * FEX + (tx + 1), l = ty * FLX + tx;
-        const int bf = k % 3;
-        const T r0 = sr[bf][c], s0 = ss[bf][c], t0 = stt[bf][c];
-        T tr = r0, ts = s0, tt = t0;
-        const T Lv = sL[k & 1][l];
-        if (i < M - 1) tr = tr + a12 * (Lv - sL[k & 1][l + 1]);
-        if (j < N - 1) ts = ts + a12 * (Lv - sL[k & 1][l + FLX]);
-        if (k < Z - 1) tt = tt + a12 * (Lv - sL[(k + 1) & 1][l]);
-        const T nrm = sqrt(tr * tr + ts * ts + tt * tt);
-        const T den = nrm > (T)1 ? nrm : (T)1;
-        if (i < M - 1) { const T on = tr / den; std_(rB, v, on + g * (on - from_raw<T, D>(co))); std_(o, v, on); }
-        else std_(rB, v, r0);
-        if (j < N - 1) { const T pn = ts / den; std_(sB, v, pn + g * (pn - from_raw<T, D>(cp))); std_(p, v, pn); }
-        else std_(sB, v, s0);
-        if (k < Z - 1) { const T qn = tt / den; std_(tB, v, qn + g * (qn - from_raw<T, D>(cq))); std_(q, v, qn); }
-        else std_(tB, v, t0);
+        if (nx) form(rn, sn, tn, t, Ln, hLn, htn, ht);
+        if (k + 2 < Z && k + 1 < k1) fetch(k + 2);
+        // dual step and projection (FGP_operator_LT_Pp)
+#pragma unroll
+        for (int a = 0; a < FGR; ++a) {
+            const T right = lane_above(L[a], lane_value(hL, 1 + a));
+            if (i >= M || j0 + a >= N) continue;
+            T tr = r[a], ts = s[a], tt = t[a];
+            if (i < M - 1) tr = tr + a12 * (L[a] - right);
+            if (j0 + a < N - 1) ts = ts + a12 * (L[a] - L[a + 1]);
+            if (nx) tt = tt + a12 * (L[a] - Ln[a]);
+            const T nrm = sqrt(tr * tr + ts * ts + tt * tt);
+            const T den = nrm > (T)1 ? nrm : (T)1;
+            // (the faces past the last planes stay zero)
+            const int64_t v = row(k, j0 + a);
+            std_(rN + v, ic, i < M - 1 ? tr / den : (T)0);
+            std_(sN + v, ic, j0 + a < N - 1 ? ts / den : (T)0);
+            std_(tN + v, ic, nx ? tt / den : (T)0);
+        }
+#pragma unroll
+        for (int a = 0; a <= FGR; ++a) { r[a] = rn[a]; s[a] = sn[a]; t[a] = tn[a]; L[a] = Ln[a]; }
+        hL = hLn; ht = htn;
     }
 }
 
@@ -611,29 +635,51 @@ static ct_status run_fgp(ct_context *ctx, int M, int N, int Z, void *vol, double
     ct_status st;
     // (the step keeps in-slice offsets in 32 bits)
     if ((int64_t)M * N >= (1ll << 31)) return fail(ctx, CT_ERR_OVERFLOW, "fgp: slice of 2^31 voxels or more");
-    // two sets of duals (read one, write the other) and the momentum copies
+    if (niter == 0) return CT_OK;   // zero duals: L is the volume itself
+    // the projected duals of three iterations: two read, one written
     D *w = (D *)slot(ctx, SLOT_FGP, sizeof(D) * V * 9, &st);
     if (!w) return st;
-    D *dual[2][3] = {{w, w + V, w + 2 * V}, {w + 6 * V, w + 7 * V, w + 8 * V}};
-    D *o = w + 3 * V, *p = w + 4 * V, *q = w + 5 * V;
-    st = launch_fill(ctx, w, dtype_of<D>(), V * 9, 0.0);
-    if (st != CT_OK) return st;
+    auto dual = [&](int it, int c) { return w + (int64_t)(it % 3 * 3 + c) * V; };
     dim3 b(256), gr((M + 255) / 256, N, Z);
-    dim3 fb(FGX, FGY), fg((M + FGX - 1) / FGX, (N + FGY - 1) / FGY, (Z + FGZ - 1) / FGZ);
+    const int lx = M > 128 ? 2 : M > 64 ? 1 : 0;   // FGW >> lx waves in y
+    // rows per wave: 8 (fewer border rows) on large FP32 volumes, where the
+    // bytes count (20 iterations at 512^3: 21.9 ms against 22.8 with 4, 23.4
+    // with 12); 4 (more waves, fewer registers) elsewhere (256^3 in FP32 3.0 ms
+    // against 3.2, 65 x 60 x 50 216 us against 361; FP16 383 x 365 x 300 6.9
+    // ms with either)
+    const bool tall = sizeof(D) == 4 && V >= (1 << 25);
+    const int rows = tall ? 8 : 4;
+    const int tx = (M + (64 << lx) - 1) / (64 << lx), ty = (N + (FGW >> lx) * rows - 1) / ((FGW >> lx) * rows);
+    // slices per workgroup: 32 (a chunk reads two border slices more), fewer on
+    // volumes that would not give eight workgroups per CU (FP16 257 x 211 x
+    // 190: 2.0 ms with 32, 1.6 with 8)
+    int zc = 32;
+    while (zc > 4 && (int64_t)tx * ty * ((Z + zc - 1) / zc) < 2048) zc >>= 1;
+    dim3 fb(64, FGW), fg(tx, ty, (Z + zc - 1) / zc);
     const T lam = (T)lambda;
     const T a12 = (T)1 / (lam * (T)12);
-    T tk1 = 1;
+    T tk1 = 1, g = 0;
     for (int it = 0; it < niter; ++it) {
-        const T tk = ((T)1 + std::sqrt((T)1 + (T)4 * tk1 * tk1)) / (T)2;
-        const T g = (tk1 - (T)1) / tk;
         ProfScope ps(ctx, CT_K_FGP);
-        D *const *A = dual[it & 1], *const *B = dual[(it + 1) & 1];
-        hipLaunchKernelGGL((k_fgp_step<S, T, D>), fg, fb, 0, ctx->stream, (const S *)vol, (const D *)A[0],
-                           (const D *)A[1], (const D *)A[2], B[0], B[1], B[2], o, p, q, M, N, Z, lam, g, a12);
+        auto step = [&](auto first) {
+            constexpr int F = decltype(first)::value;
+            constexpr int TALL = sizeof(D) == 4 ? 8 : 4;
+            hipLaunchKernelGGL((tall ? k_fgp_step<S, T, D, F, TALL> : k_fgp_step<S, T, D, F, 4>), fg, fb, 0, ctx->stream, (const S *)vol,
+                               (const D *)dual(it + 2, 0), (const D *)dual(it + 2, 1), (const D *)dual(it + 2, 2),
+                               (const D *)dual(it + 1, 0), (const D *)dual(it + 1, 1), (const D *)dual(it + 1, 2),
+                               dual(it, 0), dual(it, 1), dual(it, 2), M, N, Z, lx, zc, lam, g, a12);
+        };
+        if (it == 0) step(std::integral_constant<int, 2>());
+        else if (it == 1) step(std::integral_constant<int, 1>());
+        else step(std::integral_constant<int, 0>());
+        // momentum factor of the point this iteration's result enters
+        const T tk = ((T)1 + std::sqrt((T)1 + (T)4 * tk1 * tk1)) / (T)2;
+        g = (tk1 - (T)1) / tk;
         tk1 = tk;
     }
-    hipLaunchKernelGGL((k_fgp_L<S, T, D>), gr, b, 0, ctx->stream, (const S *)vol, (const D *)o, (const D *)p,
-                       (const D *)q, (S *)vol, (T *)nullptr, M, N, Z, lam);
+    hipLaunchKernelGGL((k_fgp_L<S, T, D>), gr, b, 0, ctx->stream, (const S *)vol, (const D *)dual(niter + 2, 0),
+                       (const D *)dual(niter + 2, 1), (const D *)dual(niter + 2, 2), (S *)vol, (T *)nullptr, M, N, Z,
+                       lam);
     return launch_check(ctx, "fgp");
 }
 

@@ -609,6 +609,26 @@ def test_ramp_filter_non_power_of_two(ctx):
     assert rel(got, ref) <= 1e-5
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 4, 63), (5, 5, 64), (9, 8, 65), (33, 9, 128), (4, 17, 129),
+                                   (3, 33, 257)])
+@pytest.mark.parametrize("niter", [0, 1, 2, 3, 6])
+def test_tv_fgp_tile_edges(ctx, shape, niter):
+    """Shapes around the step's 64-column waves, 4-row strips and slice chunks,
+    and the first iterations (no duals, one set, two): FP32 bit-identical to
+    the oracle, FP16 within its storage rounding of the FP32 result on the
+    stored input."""
+    b = np.random.default_rng(11).random(shape).astype(np.float16)
+    ref = orc.tv_fgp(b.astype(np.float32), 0.004, niter, prec=32)
+    v = dev(b.astype(np.float32))
+    ctx.tv_fgp(v, 0.004, niter)
+    assert np.array_equal(host(v), ref.astype(np.float64))
+    h = dev(b, torch.float16)
+    ctx.tv_fgp(h, 0.004, niter)
+    # half an ulp of values below 2 for the result, and 16-bit duals of the
+    # unit ball (2^-11 each, six terms, momentum at most doubling them) times lambda
+    assert float(np.abs(host(h) - ref).max()) <= 2.0 ** -11 + 0.004 * 12 * 2.0 ** -11 * (1 + niter)
+
+
 @pytest.mark.parametrize("ncols", [1, 3, 129, 255, 257, 513, 720, 1025, 2047])
 def test_ramp_filter_transform_lengths(ctx, ncols):
     """Row lengths around the transform lengths 2^9..2^12, whose taps' spectrum
