@@ -308,6 +308,22 @@ def test_column_walk_row_blocks(ctx, nrows, dt):
     assert abs(data - want) <= 4e-5 * want
 
 
+@pytest.mark.parametrize("nrows,nsources", [(96, 1), (129, 1), (270, 1), (40, 3)])
+def test_objective_column_walk(ctx, nrows, nsources):
+    """The objective of scans large enough for the column walk (2^25 ray and
+    plane pairs), rows in blocks of 128 and 256 with part blocks, and several
+    sources: the residual's 1e-5 bar on Ax doubled, as it enters squared and
+    b = Ax/2 + 0.01."""
+    g = Geometry(nx=64, ny=60, nz=52, vx=1.0, ncols=100, nrows=nrows, du=1.0, dv=90.0 / nrows, nviews=70,
+                 nsources=nsources, src_z0=-4.0 * (nsources - 1), src_dz=8.0)
+    x = phantom(g, seed=5, scale=0.6).numpy()
+    ref = orc.forward(g, x, prec=32)
+    meas = (0.5 * ref + 0.01).astype(np.float32)
+    data, _, _ = ctx.objective(g, dev(x), dev(meas))
+    want = float(((ref.astype(np.float64) - meas) ** 2).sum())
+    assert abs(data - want) <= 4e-5 * want
+
+
 @pytest.mark.parametrize("nz,nviews,kw", [(9, 1, {}), (9, 2, {}), (17, 67, {}), (7, 5, dict(nsources=3, src_z0=-4.0,
                                                                                             src_dz=4.0))])
 def test_adjoint_view_parts(ctx, nz, nviews, kw):
