@@ -224,6 +224,27 @@ static ct_status sweep(ct_context *ctx, const ct_geometry &g, void *vol, ct_dtyp
         if (tr && (st = launch_zq_transpose(ctx, volt, vdt, volq, g.nx, g.ny, g.nz, false)) != CT_OK) return st;
         return launch_zq_unpack(ctx, volq, vdt, vol, g.nx, g.ny, g.nz);
     }
+    if (planar_sweep_fits(ctx, g, vdt, subset)) {
+        // fan and parallel beam with the rows at the slice centres: the sweep
+        // runs on a z-fastest copy of the volume
+        void *volz = slot(ctx, SLOT_ZQVOL, (size_t)vox(&g) * dtype_size(vdt), &st);
+        if (!volz) return st;
+        if ((st = launch_zfast(ctx, vol, vdt, volz, g.nx, g.ny, g.nz, true)) != CT_OK) return st;
+        auto step = [&](int first, int stride, int cnt) {
+            ct_status s2 = launch_planar_corr(ctx, g, volz, vdt, (float *)corr, meas, mdt, first, stride, cnt);
+            if (s2 != CT_OK) return s2;
+            return launch_planar_update(ctx, g, volz, vdt, (const float *)corr, first, stride, cnt, beta);
+        };
+        if (order == CT_ORDER_INTERLEAVED && subset > 1) {
+            const int nsub = (nv + subset - 1) / subset;
+            for (int s = 0; s < nsub; ++s)
+                if ((st = step(s, nsub, (nv - s + nsub - 1) / nsub)) != CT_OK) return st;
+        } else {
+            for (int p0 = 0; p0 < nv; p0 += subset)
+                if ((st = step(p0, 1, std::min(subset, nv - p0))) != CT_OK) return st;
+        }
+        return launch_zfast(ctx, volz, vdt, vol, g.nx, g.ny, g.nz, false);
+    }
     if (order == CT_ORDER_INTERLEAVED && subset > 1) {
         const int nsub = (nv + subset - 1) / subset;
         for (int s = 0; s < nsub; ++s) {

@@ -347,6 +347,17 @@ ct_status launch_correction_zq(ct_context *ctx, const ct_geometry &g, const void
                                bool tr = false);
 ct_status launch_voxel_bp_zq(ct_context *ctx, const ct_geometry &g, void *volq, ct_dtype vdt, const void *corr,
                              int32_t first, int32_t stride, int32_t nv, double beta, bool tr = false);
+// Planar sweep (fan or parallel beam with the rows at the slice centres): the
+// volume in the z-fastest layout [y][x][z], corrections [image][column][row]
+bool planar_sweep_fits(const ct_context *ctx, const ct_geometry &g, ct_dtype vdt, int subset);
+ct_status launch_zfast(ct_context *ctx, const void *in, ct_dtype dt, void *out, int M, int N, int Z, bool to_zfast);
+ct_status launch_planar_corr(ct_context *ctx, const ct_geometry &g, const void *volz, ct_dtype vdt, float *corr,
+                             const void *meas, ct_dtype mdt, int32_t first, int32_t stride, int32_t nv);
+ct_status launch_planar_update(ct_context *ctx, const ct_geometry &g, void *volz, ct_dtype vdt, const float *corr,
+                               int32_t first, int32_t stride, int32_t nv, double beta);
+// log2 of the lanes that share a column's slices: the power of two from 64 to
+// 256 that holds them
+inline int planar_zshift(int Z) { return Z <= 64 ? 6 : Z <= 128 ? 7 : 8; }
 ct_status launch_forward_mv(ct_context *ctx, const ct_geometry &g, const void *vol, ct_dtype vdt, void *out,
                             ct_dtype odt, const void *meas, ct_dtype mdt, int32_t first, int32_t stride,
                             int32_t nv, int cmd, int32_t mv0);

@@ -151,6 +151,44 @@ ct_status launch_zq_transpose(ct_context *ctx, const void *in, ct_dtype dt, void
     return launch_check(ctx, "z-quad transpose");
 }
 
+// [z][y][x] <-> [y][x][z]: per y a Z x M matrix is transposed, in 32 x 32 tiles
+// through LDS.
+template <typename S>
+__global__ __launch_bounds__(256) void k_zfast(const S *__restrict__ in, S *__restrict__ out, int M, int N, int Z,
+                                               int to) {
+    __shared__ S tile[32][33];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5, y = blockIdx.z;
+    const int x0 = blockIdx.x * 32, z0 = blockIdx.y * 32;
+    const int64_t MN = (int64_t)M * N;
+#pragma unroll
+    for (int k = 0; k < 32; k += 8) {
+        const int z = z0 + (to ? ty + k : tx), x = x0 + (to ? tx : ty + k);
+        if (z < Z && x < M)
+            tile[ty + k][tx] = in[to ? (int64_t)z * MN + (int64_t)y * M + x : ((int64_t)y * M + x) * Z + z];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 32; k += 8) {
+        const int z = z0 + (to ? tx : ty + k), x = x0 + (to ? ty + k : tx);
+        if (z < Z && x < M)
+            out[to ? ((int64_t)y * M + x) * Z + z : (int64_t)z * MN + (int64_t)y * M + x] = tile[tx][ty + k];
+    }
+}
+ct_status launch_zfast(ct_context *ctx, const void *in, ct_dtype dt, void *out, int M, int N, int Z, bool to_zfast) {
+    dim3 g((M + 31) / 32, (Z + 31) / 32, N), b(256);
+    switch (dt) {
+    case CT_F32:
+        hipLaunchKernelGGL(k_zfast<uint32_t>, g, b, 0, ctx->stream, (const uint32_t *)in, (uint32_t *)out, M, N, Z, (int)to_zfast);
+        break;
+    case CT_F16:
+    case CT_BF16:
+        hipLaunchKernelGGL(k_zfast<uint16_t>, g, b, 0, ctx->stream, (const uint16_t *)in, (uint16_t *)out, M, N, Z, (int)to_zfast);
+        break;
+    default: return fail(ctx, CT_ERR_DTYPE, "z-fastest copy: unsupported dtype");
+    }
+    return launch_check(ctx, "z-fastest copy");
+}
+
 template <typename SO>
 __global__ __launch_bounds__(256) void k_zq_unpack_f64(const double *__restrict__ in, SO *__restrict__ out, int M, int N,
                                                        int Z) {

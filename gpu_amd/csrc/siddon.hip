@@ -1014,6 +1014,118 @@ __global__ __launch_bounds__(RW) void k_project_col(DGeo<float> d, const float *
     if constexpr (CMD != 2) St<SO>::st(out, (int64_t)img * P + pix, r);
 }
 
+// SART correction of fan- and parallel-beam views whose detector rows lie at
+// the slice centres (planar_sweep_fits): a ray then stays in its row's slice,
+// and all rows of a detector column cross the same x/y cells over the same
+// alphas.  The volume is in the z-fastest layout [y][x][z], so a cell's slices
+// are contiguous: zw lanes (a power of two from 64 to 256) take one column's
+// slices, the column's cells and alpha lengths are listed once in LDS (the
+// merge of k_project_col, clipped to the ray's [alpha_min, alpha_max]), and a
+// segment costs every lane one coalesced load and one FMA, whatever the ray's
+// direction.  Batches of 16 segments are summed in FP32 and the batch sums
+// Kahan-compensated, as in the other walks.  The corrections are stored
+// [image][column][row], as k_planar_update reads them.
+//
+// Bound by L2: 512 x 512 x 256 / 1024 x 256 0.052 ms per view, against 0.28 ms
+// for one per-ray walk per lane.
+template <typename SV, typename SM>
+__global__ __launch_bounds__(256) void k_planar_corr(DGeo<float> d, const float *__restrict__ ang,
+                                                     const SV *__restrict__ fz, float *__restrict__ corr,
+                                                     const SM *__restrict__ meas, int first, int stride, int zsh) {
+    extern __shared__ __align__(16) unsigned char pl_smem[];
+    constexpr int B = 16, ES = (int)sizeof(SV);
+    const int zw = 1 << zsh, cpw = 256 >> zsh;
+    const int LE = (d.M + d.N + B) & ~(B - 1);           // list entries of a column, padded (at most M + N - 1 used)
+    const int tid = threadIdx.x, c = tid >> zsh, zt = tid & (zw - 1);
+    const int3 t = xcd_tile();
+    const int col = t.x * cpw + c, z = t.y * zw + zt, img = t.z;
+    const int v = first + img * stride;
+    const float s = ang[2 * v], cs = ang[2 * v + 1];
+    uint2 *const list = reinterpret_cast<uint2 *>(pl_smem) + (size_t)c * LE;   // (alpha length, byte offset of the cell)
+    FastWalk<1> fw;
+    // (the column's rays differ in the slice alone)
+    const bool hit = col < d.R && fw.init(d, s, cs, col, t.y * zw, 0);
+    int KP = 0;
+    if (hit) {
+        const float u = d.ymin + (float)col * d.du;
+        const float x1x = d.dod * cs - u * s, x1y = d.dod * s + u * cs;
+        float x2x, x2y, x2z;
+        ray_source(d, s, cs, u, 0.0f, 0, x2x, x2y, x2z);
+        const int sgx = (x1x < x2x) ? 1 : ((x1x > x2x) ? -1 : 0), sgy = (x1y < x2y) ? 1 : ((x1y > x2y) ? -1 : 0);
+        const PlaneAxis X = plane_axis(d.vx, d.ivx, d.bx, x1x, 1.0f / (x2x - x1x), sgx, d.vx * 1e-6f > fabsf(x1x - x2x));
+        const PlaneAxis Y = plane_axis(d.vy, d.ivy, d.by, x1y, 1.0f / (x2y - x1y), sgy, d.vy * 1e-6f > fabsf(x1y - x2y));
+        const float lo = fw.ac, hi = fw.amax;
+        float nf;
+        int vi0 = X.i0, vj0 = Y.i0, NX = 0, NY = 0;
+        if (!X.par) {
+            vi0 = FastWalk<1>::restart_axis(X.k, X.b0, (float)sgx, nf, lo, d.M);
+            NX = max((FastWalk<1>::restart_axis(X.k, X.b0, (float)sgx, nf, hi, d.M) - vi0) * sgx, 0);
+        }
+        if (!Y.par) {
+            vj0 = FastWalk<1>::restart_axis(Y.k, Y.b0, (float)sgy, nf, lo, d.N);
+            NY = max((FastWalk<1>::restart_axis(Y.k, Y.b0, (float)sgy, nf, hi, d.N) - vj0) * sgy, 0);
+        }
+        const int K = NX + NY;                  // crossings; entry K ends at hi
+        KP = (K + B) / B * B;
+        const float px0 = (float)(vi0 + (sgx > 0)), py0 = (float)(vj0 + (sgy > 0));
+        const float fsx = (float)sgx, fsy = (float)sgy;
+        auto XA = [&](int i) { return fmaf(fmaf((float)i, fsx, px0), X.k, X.b0); };
+        auto YA = [&](int j) { return fmaf(fmaf((float)j, fsy, py0), Y.k, Y.b0); };
+        const int C = (KP + zw - 1) >> zsh, e0 = zt * C;
+        if (e0 < KP) {
+            const int ee = min(e0, K);
+            int ilo = max(0, ee - NY), ihi = min(ee, NX);
+            while (ilo < ihi) {
+                const int mid = (ilo + ihi) >> 1;
+                if (XA(mid) <= YA(ee - mid - 1)) ilo = mid + 1;
+                else ihi = mid;
+            }
+            int i = ilo, j = ee - ilo;
+            float ap = lo;
+            if (e0 > K) ap = hi;
+            else if (ee > 0)
+                ap = __builtin_amdgcn_fmed3f(fmaxf(i > 0 ? XA(i - 1) : -__builtin_inff(), j > 0 ? YA(j - 1) : -__builtin_inff()), lo, hi);
+            for (int e = e0; e < min(e0 + C, KP); ++e) {
+                const unsigned off = ((unsigned)(vj0 + j * sgy) * (unsigned)d.M + (unsigned)(vi0 + i * sgx)) * (unsigned)d.Z * (unsigned)ES;
+                float a = hi;
+                if (e < K) {
+                    if (i < NX && (j >= NY || XA(i) <= YA(j))) { a = XA(i); ++i; }
+                    else { a = YA(j); ++j; }
+                    a = __builtin_amdgcn_fmed3f(a, lo, hi);
+                }
+                list[e] = make_uint2(__float_as_uint(a - ap), off);
+                ap = a;
+            }
+        }
+    }
+    __syncthreads();
+    if (col >= d.R) return;
+    float sum = 0.0f, comp = 0.0f;
+    const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(fz, (uint32_t)d.M * (uint32_t)d.N * (uint32_t)d.Z * (uint32_t)ES);
+    const uint32_t zo = (uint32_t)z * (uint32_t)ES;
+    for (int e = 0; e < KP; e += B) {
+        float dl[B], fv[B];
+#pragma unroll
+        for (int k = 0; k < B; k += 2) {
+            const uint4 w = *reinterpret_cast<const uint4 *>(list + e + k);
+            dl[k] = __uint_as_float(w.x); dl[k + 1] = __uint_as_float(w.z);
+            fv[k] = bload<SV>(rs, w.y + zo);
+            fv[k + 1] = bload<SV>(rs, w.w + zo);
+        }
+        float ps = dl[0] * fv[0];
+#pragma unroll
+        for (int k = 1; k < B; ++k) ps = fmaf(dl[k], fv[k], ps);
+        const float y = ps - comp, tt = sum + y;
+        comp = (tt - sum) - y;
+        sum = tt;
+    }
+    if (z >= d.Z) return;
+    float r = 0.0f;
+    if (hit && !(fw.len < d.vz * 1e-6f))
+        r = ((float)ldf(meas, ((int64_t)v * d.ZP + z) * d.R + col) - (sum - comp) * fw.dist) / fw.len;
+    corr[((int64_t)img * d.R + col) * d.Z + z] = r;
+}
+
 // Data fidelity sum (Ax - b)^2 fused into the ray traversal: Ax never goes to
 // memory.  Geometries that admit the column walk take it (CMD 2 of
 // k_project_col); this per-ray form serves the others, exact mode and FP64.
@@ -1947,6 +2059,44 @@ ct_status launch_correction_zq(ct_context *ctx, const ct_geometry &g, const void
     default: break;
     }
     return fail(ctx, CT_ERR_DTYPE, "z-quad correction: unsupported volume dtype");
+}
+
+template <typename SV>
+static ct_status planar_corr_meas(ct_context *ctx, const DGeo<float> &d, const float *ang, const void *volz, float *corr,
+                                  const void *meas, ct_dtype mdt, int first, int stride, int nv) {
+    const int zsh = planar_zshift(d.Z);
+    const int cpw = 256 >> zsh, LE = (d.M + d.N + 16) & ~15;
+    dim3 grid((d.R + cpw - 1) / cpw, (d.Z + (1 << zsh) - 1) >> zsh, nv);
+    const size_t lds = sizeof(uint2) * (size_t)LE * cpw;
+    auto go = [&](auto m) {
+        using SM = decltype(m);
+        hipLaunchKernelGGL((k_planar_corr<SV, SM>), grid, dim3(256), lds, ctx->stream, d, ang, (const SV *)volz, corr,
+                           (const SM *)meas, first, stride, zsh);
+    };
+    switch (mdt) {
+    case CT_F32: go(float()); break;
+    case CT_F16: go(__half()); break;
+    case CT_BF16: go(__hip_bfloat16()); break;
+    case CT_F64: go(double()); break;
+    }
+    return launch_check(ctx, "planar correction");
+}
+
+ct_status launch_planar_corr(ct_context *ctx, const ct_geometry &g, const void *volz, ct_dtype vdt, float *corr,
+                             const void *meas, ct_dtype mdt, int32_t first, int32_t stride, int32_t nv) {
+    if (nv <= 0) return CT_OK;
+    ct_status st;
+    const float *ang = (const float *)angle_table(ctx, g, false, false, &st);
+    if (!ang) return st;
+    const DGeo<float> d = derive<float>(g);
+    ProfScope ps(ctx, CT_K_FORWARD);
+    switch (vdt) {
+    case CT_F32: return planar_corr_meas<float>(ctx, d, ang, volz, corr, meas, mdt, first, stride, nv);
+    case CT_F16: return planar_corr_meas<__half>(ctx, d, ang, volz, corr, meas, mdt, first, stride, nv);
+    case CT_BF16: return planar_corr_meas<__hip_bfloat16>(ctx, d, ang, volz, corr, meas, mdt, first, stride, nv);
+    default: break;
+    }
+    return fail(ctx, CT_ERR_DTYPE, "planar correction: unsupported volume dtype");
 }
 
 // The sweep walks views whose rays run along y on the transposed z-quad

@@ -308,6 +308,29 @@ def test_column_walk_row_blocks(ctx, nrows, dt):
     assert abs(data - want) <= 4e-5 * want
 
 
+@pytest.mark.parametrize("nz,nviews,subset,order", [(1, 3, 1, "ascending"), (5, 19, 18, "interleaved"),
+                                                    (64, 4, 1, "ascending"), (65, 4, 2, "ascending"),
+                                                    (129, 3, 1, "ascending"), (257, 2, 1, "ascending")])
+@pytest.mark.parametrize("style,du", [(1, 1.1), (2, 0.45)])
+def test_planar_sweep(ctx, nz, nviews, subset, order, style, du):
+    """Fan- and parallel-beam sweeps in the z-fastest layout: slice counts
+    around the lanes per column (64, 128, 256), more views per update than are
+    listed at once, and fine columns (more than four chords per voxel), at the
+    1e-4 reconstruction bar against the FP32 oracle; 16-bit storage at the
+    rounding of one stored update per subset."""
+    g = small_geom(nx=21, ny=26, nz=nz, nrows=nz, dv=1.0, ncols=int(40 / du), du=du, nviews=nviews, style=style)
+    x = phantom(g, seed=2, scale=0.3).numpy()
+    b = orc.forward(g, x, prec=32)
+    x0 = (0.7 * x + 0.004).astype(np.float16).astype(np.float32)
+    ref = orc.sart_sweep(g, x0, b, beta=0.8, subset=subset, order=order, prec=32)
+    v = dev(x0)
+    ctx.sart_sweep(g, v, dev(b), beta=0.8, subset=subset, order=order)
+    assert rel(host(v), ref) <= 1e-4
+    h = dev(x0, torch.float16)
+    ctx.sart_sweep(g, h, dev(b), beta=0.8, subset=subset, order=order)
+    assert rel(host(h), ref) <= 1e-3 * -(-nviews // subset)
+
+
 @pytest.mark.parametrize("nrows,nsources", [(96, 1), (129, 1), (270, 1), (40, 3)])
 def test_objective_column_walk(ctx, nrows, nsources):
     """The objective of scans large enough for the column walk (2^25 ray and
