@@ -199,8 +199,8 @@ static ct_status sweep(ct_context *ctx, const ct_geometry &g, void *vol, ct_dtyp
         void *volt = nullptr;
         bool tr = false;
         auto step = [&](int first, int stride, int cnt) {
-            const bool want = subset == 1 || cnt == 1 ? sweep_view_transposed(g, first)
-                                                      : sweep_view_transposed(g, first + stride * (cnt / 2));
+            const bool want = subset == 1 || cnt == 1 ? sweep_view_transposed(g, vdt, first, cnt)
+                                                      : sweep_view_transposed(g, vdt, first + stride * (cnt / 2), cnt);
             if (want != tr) {
                 if (!volt && !(volt = slot(ctx, SLOT_ZQVOL_T, bytes, &st))) return st;
                 ct_status s0 = want ? launch_zq_transpose(ctx, volq, vdt, volt, g.nx, g.ny, g.nz, true)

@@ -338,9 +338,10 @@ ct_status launch_zq_unpack_f64(ct_context *ctx, const double *accq, void *vol, c
 ct_status launch_zq_transpose(ct_context *ctx, const void *in, ct_dtype dt, void *out, int M, int N, int Z,
                               bool to_tr);
 bool sweep_zq_eligible(const ct_context *ctx, const ct_geometry &g, ct_dtype vdt, int subset);
-// whether the sweep runs view v's correction and update on the transposed
-// z-quad layout (its rays run along y and the column walk is admitted)
-bool sweep_view_transposed(const ct_geometry &g, int v);
+// whether the sweep runs the correction and update of nv views around view v
+// on the transposed z-quad layout (its rays run along y and the launch takes
+// the column walk)
+bool sweep_view_transposed(const ct_geometry &g, ct_dtype vdt, int v, int nv);
 // tr: the volume is in the transposed z-quad layout
 ct_status launch_correction_zq(ct_context *ctx, const ct_geometry &g, const void *volq, ct_dtype vdt, float *corr,
                                const void *meas, ct_dtype mdt, int32_t first, int32_t stride, int32_t nv,
@@ -355,9 +356,15 @@ ct_status launch_planar_corr(ct_context *ctx, const ct_geometry &g, const void *
                              const void *meas, ct_dtype mdt, int32_t first, int32_t stride, int32_t nv);
 ct_status launch_planar_update(ct_context *ctx, const ct_geometry &g, void *volz, ct_dtype vdt, const float *corr,
                                int32_t first, int32_t stride, int32_t nv, double beta);
-// log2 of the lanes that share a column's slices: the power of two from 64 to
-// 256 that holds them
-inline int planar_zshift(int Z) { return Z <= 64 ? 6 : Z <= 128 ? 7 : 8; }
+// log2 of the lanes that share a column's slices: of 256, 128 and 64 the one
+// that leaves the fewest without a slice, the larger at a tie (258 slices: 320
+// lanes in five blocks of 64, where two of 256 left half idle)
+inline int planar_zshift(int Z) {
+    int best = 8;
+    for (int s = 7; s >= 6; --s)
+        if ((Z + (1 << s) - 1) >> s << s < (Z + (1 << best) - 1) >> best << best) best = s;
+    return best;
+}
 ct_status launch_forward_mv(ct_context *ctx, const ct_geometry &g, const void *vol, ct_dtype vdt, void *out,
                             ct_dtype odt, const void *meas, ct_dtype mdt, int32_t first, int32_t stride,
                             int32_t nv, int cmd, int32_t mv0);

@@ -623,7 +623,7 @@ __global__ __launch_bounds__(256) void k_project_zq(DGeo<float> d, const float *
 // three beam styles those points share their x and y: the rays of a column
 // lie in one vertical plane and cross the x and y planes at the same alpha
 // (fma(n, k, b0) over the same k and b0, so the same FP32 numbers).  A
-// workgroup takes 256 rows of one column and merges the column's x and y
+// workgroup takes 256 rows (or 128) of one column and merges the column's x and y
 // crossings once into an LDS list; each list segment is one x/y voxel, and at
 // a segment all 256 rays read that voxel column of z, within a window the
 // list also records (the extreme rows at the segment's ends, one voxel of
@@ -683,9 +683,10 @@ template <typename SV> struct StageOf { using type = float; };
 template <> struct StageOf<__half> { using type = _Float16; };
 
 // fq is the volume in the z-quad layout and ft in its lateral transpose
-// [z/4][x][y][z%4]; a view reads the one along whose fast axis its rays run
-// (col_walk_view: the staged quads of consecutive segments then share cache
-// lines), so one launch takes views of both directions.
+// [z/4][x][y][z%4], either of them null; a view reads the one along whose fast
+// axis its rays run (col_walk_view: the staged quads of consecutive segments
+// then share cache lines) if both are there, so one launch takes views of both
+// directions.
 template <typename SV, typename SO, typename SM, int CMD, int RW>
 __global__ __launch_bounds__(RW) void k_project_col(DGeo<float> d, const float *__restrict__ ang,
                                                           const SV *__restrict__ fq, const SV *__restrict__ ft,
@@ -710,7 +711,7 @@ __global__ __launch_bounds__(RW) void k_project_col(DGeo<float> d, const float *
     const int q = img / d.NS, src = img - q * d.NS;
     const int v = first + q * stride;
     const float s = ang[2 * v], c = ang[2 * v + 1];
-    const bool tr = !col_along_x(c);
+    const bool tr = !fq || (ft && !col_along_x(c));
     const unsigned M = d.M, MN = (unsigned)d.M * (unsigned)d.N;
     const int ZQ4 = (d.Z + 3) >> 2;                        // quads per (x, y)
     const unsigned QS = MN * 4u * (unsigned)ES;            // bytes between z-quad planes
@@ -1597,13 +1598,18 @@ static bool adj_gather_fits(const DGeo<float> &d) {
 // fan and parallel rays keep their row height.  One voxel of the segment's
 // own z travel, one of rounding margin on each side and the quad alignment
 // are added.
-// Of the two workgroup sizes the one with fewer lanes past the last row, and
-// 256 rows at a tie: at 512^3 / 1024^2, where both fill, a view takes 0.34 ms
-// with 256 and 0.36 ms with 128 (FP32; each workgroup makes its own list).
-// With 128 an FP16 correction of 1000 x 830 on 500 x 468 x 391 takes 0.26 ms
-// against 0.28, the gradient of 90 views of 96^2 on 64^3 163 us against 217,
-// and the 128^3 / 256^2 sweep in subsets of 20, whose 256 rows overrun the
-// window, 2.48 ms against 2.70 with the per-ray walk.
+// Of the two workgroup sizes 256, unless 128 leaves enough fewer lanes past
+// the last row to pay for its second list: any on 16-bit volumes, a quarter on
+// FP32 ones, whose staging weighs more (corrections of 24 views, FP32: 840
+// rows on 420^3, 7/8 of the lanes, 11.2 -> 11.7 ms with 128; 560 on 280^3, 5/6,
+// 4.1 -> 4.0; FP16: 640 on 320^3, 5/6, 4.7 -> 4.4; gradient of 90 views of 96
+// rows on 64^3 217 -> 163 us).  Where 256 rows overrun the window, 128 serve;
+// not for corrections of FP32 volumes beyond the 32 MB of the XCDs' L2, nor on
+// 16-bit ones of fewer than four images or with more than an eighth of the lanes
+// past the last row: the per-ray walk is then the faster one (dv/vz = 1, FP32,
+// four views at a time: 200^3 0.82 -> 0.78 ms by column, 512^3 10.4 -> 11.3;
+// FP16: 512^3 10.2 -> 9.7, one at a time 4.4 -> 5.4; 420^3 with 504 rows
+// 5.5 -> 5.0, six at a time with 525 rows 8.5 -> 9.2).
 struct ColPlan { int rows, nq; };   // nq 0: the walk is not admitted
 static int col_quads(const DGeo<float> &d, int rw, int max_nq) {
     if ((d.ZP + rw - 1) / rw > 65535) return 0;
@@ -1621,8 +1627,11 @@ static int col_quads(const DGeo<float> &d, int rw, int max_nq) {
     const double nq = std::ceil((span + 8.0) / 4.0);
     return nq >= 1.0 && nq <= max_nq ? (int)nq : 0;
 }
-static ColPlan col_plan(const DGeo<float> &d) {
-    const ColPlan none = {0, 0};
+// The windows of 256 and 128 rows a launch would stage; 0 where they are not
+// admitted.
+struct ColQuads { int n256, n128; };
+static ColQuads col_fits(const DGeo<float> &d) {
+    const ColQuads none = {0, 0};
     if ((uint64_t)d.M * d.N * (uint64_t)((d.Z + 3) & ~3) * 4 >= (1ull << 31)) return none;
     double dzmax = 0.0;
     const double inplane = std::fabs((double)d.dso - (double)d.dod);
@@ -1635,10 +1644,20 @@ static ColPlan col_plan(const DGeo<float> &d) {
     if (!(dzmax / (double)d.vz < 0.9 * inplane / (std::sqrt(2.0) * vxy))) return none;
     // (the padding of col_dyn_lds keeps a workgroup under 33 KiB)
     if (col_lds_bytes(d.M, d.N) > 65536) return none;
-    const int n256 = col_quads(d, 256, col_nq<256>()), n128 = col_quads(d, 128, col_nq<128>());
+    return {col_quads(d, 256, col_nq<256>()), col_quads(d, 128, col_nq<128>())};
+}
+static ColPlan col_plan(const DGeo<float> &d, size_t es, int nimg, bool corrections) {
+    const ColPlan none = {0, 0};
+    const ColQuads q = col_fits(d);
+    const int n256 = q.n256, n128 = q.n128;
     const int pad256 = (d.ZP + 255) / 256 * 256, pad128 = (d.ZP + 127) / 128 * 128;
-    if (n128 > 0 && (n256 == 0 || pad128 < pad256)) return {128, n128};
-    return {n256 > 0 ? 256 : 0, n256};
+    if (n256 == 0) {
+        const bool ray = corrections && (es == 4 ? (uint64_t)d.M * d.N * d.Z * es > (32u << 20)
+                                                 : nimg < 4 || 8 * pad128 > 9 * d.ZP);
+        return n128 > 0 && !ray ? ColPlan{128, n128} : none;
+    }
+    if (n128 > 0 && (es == 2 ? pad128 < pad256 : 4 * pad256 >= 5 * pad128)) return {128, n128};
+    return {256, n256};
 }
 
 // Dynamic LDS of a launch: the list, padded so that a workgroup of 256 holds
@@ -1668,6 +1687,31 @@ static void launch_col_rw(ct_context *ctx, const DGeo<float> &d, int nq, const f
     }
 }
 
+// (ray, x/y plane) pairs of a launch.  The column walk's lists, barriers and
+// volume copies pay from 3 * 2^24 on, twice that for the objective, whose
+// alternative reads the linear volume.  Corrections of 24 views, FP32, one at a
+// time: 200^3 / 400^2 (2^25.9) 1.91 ms by column, 1.87 by ray, 240^3 / 480^2
+// (2^26.7) 2.48 and 2.92; four at a time: 96^3 / 192^2 (2^24.8) 0.73 and 0.71,
+// 160^3 / 256 x 192 (2^25.9) 0.45 and 0.51; eight single views of 128^3 / 204 x
+// 152 0.35 and 0.25.  Ray sums of 24 views on 96^3 with the adjoint 0.136 and
+// 0.157 ms.  Objective: 119 x 133 x 119, 6 views of 237 x 196 in FP16 (2^26.1)
+// 115 us by column, 108 by ray; 120 x 127 x 79, 20 views of 200 x 123 in FP32
+// (2^26.9) 128 and 146.
+static double col_pairs(const DGeo<float> &d, int nimg) { return (double)d.R * d.ZP * nimg * (d.M + d.N); }
+constexpr double COL_MIN = (double)(3 << 24);
+
+// The plan of corrections.  A BF16 sweep's updates are stored with a
+// dither from the low bits of their sums, so that another order of summing a ray
+// changes the volume by up to 2% of its norm in 60 views (FP16 0.3%): BF16 keeps
+// one walk at all sizes, by column wherever 256 rows fit.
+static ColPlan sweep_plan(const DGeo<float> &d, ct_dtype vdt, int nimg) {
+    if (vdt == CT_BF16) {
+        const int n = col_fits(d).n256;
+        return {n > 0 ? 256 : 0, n};
+    }
+    return col_pairs(d, nimg) >= COL_MIN ? col_plan(d, dtype_size(vdt), nimg, true) : ColPlan{0, 0};
+}
+
 // The column walk stages, per segment, one z-quad of each (x, y) on the
 // column's path; a 128-byte line holds eight neighbours along the layout's
 // fast axis, so paths that run along it use whole lines and paths across it
@@ -1694,25 +1738,27 @@ static void launch_zq(ct_context *ctx, const DGeo<float> &d, const float *ang, c
 
 // Walks the views first, first + stride, ... of a z-quad volume by column.
 // volq is in the plain layout or, with `tr`, the transposed one (each in its
-// own slot of the context).  Views that run the other way need the other copy
-// (0.17 ms at 512^3 in FP32), which pays from the first view on FP32 volumes
-// (0.59 -> 0.39 ms per view there), but for 16-bit ones, whose per-ray walk
-// is nearly as fast (358 x 342 x 339 / 718 x 707 in FP16: 0.154 -> 0.149 ms
-// per view, the copy 0.036 ms), only from eight images on; fewer take the
-// per-ray walk on volq.
+// own slot of the context); views that run the other way take the other copy.
 template <typename SV, typename SO, typename SM, int CMD>
 static ct_status launch_col(ct_context *ctx, const ct_geometry &g, const DGeo<float> &d, ColPlan cp, const float *ang,
                             const void *volq, bool tr, void *out, const void *meas, int first, int stride, int nv,
                             int mv0) {
-    const void *vols[2] = {volq, volq};
+    const void *vols[2] = {tr ? nullptr : volq, tr ? volq : nullptr};
     auto walk = [&](int q0, int n, void *o) {
         if (cp.rows == 256) launch_col_rw<SV, SO, SM, CMD, 256>(ctx, d, cp.nq, ang, vols, o, meas, first + q0 * stride, stride, mv0, n * d.NS);
         else launch_col_rw<SV, SO, SM, CMD, 128>(ctx, d, cp.nq, ang, vols, o, meas, first + q0 * stride, stride, mv0, n * d.NS);
     };
     int others = 0;
     for (int q = 0; q < nv; ++q) others += col_walk_view(g, first + q * stride) == tr;
-    if constexpr (CMD != 2 && sizeof(SV) == 2) {
-        if (others > 0 && others * d.NS < 8 && !tr) {
+    // Fewer than four images of the other direction do without the copy: in the
+    // transposed layout (which the sweep takes by the middle view) and for the
+    // objective they walk the layout that is there, in the plain one by ray
+    // (FP32, 263 x 261 x 251 / 549 x 459, three views and two: 0.19 ms, 0.23 on
+    // the layout that is there; 512^3 / 1024^2 in subsets of four 22.4 ms, 23.0
+    // with the copy).  So do all of a BF16 sweep's, at all sizes (sweep_plan).
+    const bool few = others * d.NS < 4 || (CMD == 1 && std::is_same<SV, __hip_bfloat16>::value);
+    if constexpr (CMD != 2) {
+        if (others > 0 && few && !tr) {
             const int64_t P = (int64_t)d.R * d.ZP * d.NS;
             for (int q0 = 0, q1; q0 < nv; q0 = q1) {
                 const bool w = col_walk_view(g, first + q0 * stride);
@@ -1724,7 +1770,7 @@ static ct_status launch_col(ct_context *ctx, const ct_geometry &g, const DGeo<fl
             return CT_OK;
         }
     }
-    if (others > 0) {
+    if (!few) {
         ct_status st;
         const uint64_t bytes = (uint64_t)d.M * d.N * (uint64_t)((d.Z + 3) & ~3) * sizeof(SV);
         void *t = slot(ctx, tr ? SLOT_ZQVOL : SLOT_ZQVOL_T, bytes, &st);
@@ -1747,13 +1793,11 @@ static ct_status run_residual(ct_context *ctx, const ct_geometry &g, const void 
     const int nimg = g.nviews * d.NS;
     const bool comp = std::is_same<T, float>::value && ctx->math == CT_MATH_FAST;
     if constexpr (std::is_same<T, float>::value) {
-        // the batched ray sums' column walk, on the same conditions, where
-        // the walk outweighs the copies of the volume: 2^25 (ray, x/y plane)
-        // pairs (64^3, 16 views of 102 x 96: 82 us against 80 by ray, 64 views
-        // 117 against 129; 32^3, 16 views of 51 x 48: 69 against 62)
+        // the batched ray sums' column walk where it outweighs the copies of
+        // the volume
         const uint64_t qbytes = (uint64_t)d.M * d.N * (uint64_t)((d.Z + 3) & ~3) * sizeof(SV);
-        const bool large = (double)d.R * d.ZP * nimg * (d.M + d.N) >= (double)(1 << 25);
-        const ColPlan cp = comp && large && nimg >= 4 && qbytes < (1ull << 32) ? col_plan(d) : ColPlan{0, 0};
+        const bool large = col_pairs(d, nimg) >= 2 * COL_MIN;
+        const ColPlan cp = comp && large && nimg >= 4 && qbytes < (1ull << 32) ? col_plan(d, sizeof(SV), nimg, false) : ColPlan{0, 0};
         if (cp.nq > 0) {
             const int64_t per = (int64_t)d.R * ((d.ZP + cp.rows - 1) / cp.rows);   // workgroups per image
             double *part = (double *)slot(ctx, SLOT_TMP_PROJ2, sizeof(double) * per * nimg, &st);
@@ -1835,13 +1879,13 @@ static ct_status run_forward(ct_context *ctx, const ct_geometry &g, const void *
         // admits it; otherwise one walk per ray for ray sums and each ray
         // split in two for corrections
         const uint64_t qbytes = (uint64_t)d.M * d.N * (uint64_t)((d.Z + 3) & ~3) * sizeof(SV);
-        if (comp && nimg >= 4 && qbytes < (1ull << 32)) {
+        if (comp && nimg >= 4 && qbytes < (1ull << 32) && (CMD == 1 || col_pairs(d, nimg) >= COL_MIN)) {
             void *volq = slot(ctx, SLOT_ZQVOL, qbytes, &st);
             if (!volq) return st;
             ProfScope ps(ctx, CT_K_FORWARD);   // the copy is part of the call's cost
             st = launch_zq_pack(ctx, vol, dtype_of<SV>(), volq, d.M, d.N, d.Z);
             if (st != CT_OK) return st;
-            const ColPlan cp = col_plan(d);
+            const ColPlan cp = CMD == 1 ? sweep_plan(d, dtype_of<SV>(), nimg) : col_plan(d, sizeof(SV), nimg, false);
             if (cp.nq > 0) {
                 st = launch_col<SV, SO, SM, CMD>(ctx, g, d, cp, ang, volq, false, out, meas, first, stride, nv, mv0);
                 if (st != CT_OK) return st;
@@ -2022,7 +2066,7 @@ static ct_status run_correction_zq(ct_context *ctx, const ct_geometry &g, const 
     if (!ang) return st;
     DGeo<float> d = derive<float>(g);
     ProfScope ps(ctx, CT_K_FORWARD);
-    const ColPlan cp = col_plan(d);
+    const ColPlan cp = sweep_plan(d, dtype_of<SV>(), nv * d.NS);
     if (cp.nq > 0) {
         // (a subset's views may run both ways; the update that follows works
         // on volq, so the other copy serves this correction alone)
@@ -2093,7 +2137,6 @@ ct_status launch_planar_corr(ct_context *ctx, const ct_geometry &g, const void *
     switch (vdt) {
     case CT_F32: return planar_corr_meas<float>(ctx, d, ang, volz, corr, meas, mdt, first, stride, nv);
     case CT_F16: return planar_corr_meas<__half>(ctx, d, ang, volz, corr, meas, mdt, first, stride, nv);
-    case CT_BF16: return planar_corr_meas<__hip_bfloat16>(ctx, d, ang, volz, corr, meas, mdt, first, stride, nv);
     default: break;
     }
     return fail(ctx, CT_ERR_DTYPE, "planar correction: unsupported volume dtype");
@@ -2101,8 +2144,9 @@ ct_status launch_planar_corr(ct_context *ctx, const ct_geometry &g, const void *
 
 // The sweep walks views whose rays run along y on the transposed z-quad
 // layout, so that every view takes the column walk with line-sharing staging.
-bool sweep_view_transposed(const ct_geometry &g, int v) {
-    return !col_walk_view(g, v) && col_plan(derive<float>(g)).nq > 0;
+bool sweep_view_transposed(const ct_geometry &g, ct_dtype vdt, int v, int nv) {
+    const DGeo<float> d = derive<float>(g);
+    return !col_walk_view(g, v) && sweep_plan(d, vdt, nv * d.NS).nq > 0;
 }
 
 ct_status launch_forward(ct_context *ctx, const ct_geometry &g, const void *vol, ct_dtype vdt, void *out,
@@ -2137,10 +2181,11 @@ static ct_status run_adjoint(ct_context *ctx, const ct_geometry &g, const void *
 }
 
 // Parts the gather's views are split into: enough workgroups for four per CU
-// (what the kernel's registers admit) where the tiles alone give fewer.
+// (what the kernel's registers admit) where the tiles alone give fewer.  Under
+// eight images a workgroup is done with them sooner than another launch starts.
 static int adj_parts(const DGeo<float> &d, int nv) {
     const int64_t tiles = (int64_t)((d.M + 15) / 16) * ((d.N + 15) / 16) * ((d.Z + AZR - 1) / AZR);
-    if (tiles >= 512 || nv < 2) return 1;
+    if (tiles >= 512 || nv < 2 || nv * d.NS < 8) return 1;
     const int64_t want = std::min<int64_t>((1024 + tiles - 1) / tiles, nv);
     const int64_t vpp = (nv + want - 1) / want;
     return (int)((nv + vpp - 1) / vpp);

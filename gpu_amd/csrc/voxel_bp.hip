@@ -1209,11 +1209,18 @@ __global__ __launch_bounds__(256) void k_planar_many(DGeo<float> d, const float 
 // layout: rows at the slice centres, every voxel's shadow within PMAXC columns
 // (the bound of bp_lds_fits on the voxel's diagonal), 32-bit volume offsets,
 // column indices below 2^24 and the columns' lists within the LDS.
+// BF16 volumes keep the general path: their updates are stored with a dither
+// from the low bits of W and L, which another order of the sums changes by up
+// to 1% of the volume's norm.  A single update of a few views on an FP32 volume
+// beyond the 32 MB of the L2s doesn't pay for the copies (five views, 261 x 247
+// x 258: 0.35 ms on the general path, 0.40 here; FP16 295 x 281 x 211, six views
+// 0.38 and 0.33; five views in two updates, 115 x 116 x 57, 0.14 and 0.05).
 bool planar_sweep_fits(const ct_context *ctx, const ct_geometry &g, ct_dtype vdt, int subset) {
-    if (vdt == CT_F64) return false;
+    if (vdt == CT_F64 || vdt == CT_BF16) return false;
     const DGeo<float> d = derive<float>(g);
     if (!planar_eligible(ctx, d) || subset > 65535 || d.N > 65535 || d.R >= (1 << 24)) return false;
-    if ((uint64_t)d.M * d.N * d.Z * dtype_size(vdt) >= (1ull << 32)) return false;
+    const uint64_t bytes = (uint64_t)d.M * d.N * d.Z * dtype_size(vdt);
+    if (bytes >= (1ull << 32) || (vdt == CT_F32 && g.nviews < 8 && subset >= g.nviews && bytes > (32u << 20))) return false;
     if ((size_t)8 * ((d.M + d.N + 16) & ~15) * (256 >> planar_zshift(d.Z)) > 64 * 1024) return false;
     const double xs[2] = {(double)d.bx, (double)d.bx + (double)d.M * d.vx};
     const double ys[2] = {(double)d.by, (double)d.by + (double)d.N * d.vy};
@@ -1263,7 +1270,6 @@ ct_status launch_planar_update(ct_context *ctx, const ct_geometry &g, void *volz
     switch (vdt) {
     case CT_F32: return planar_update<float>(ctx, d, ang, volz, corr, first, stride, nv, beta);
     case CT_F16: return planar_update<__half>(ctx, d, ang, volz, corr, first, stride, nv, beta);
-    case CT_BF16: return planar_update<__hip_bfloat16>(ctx, d, ang, volz, corr, first, stride, nv, beta);
     default: break;
     }
     return fail(ctx, CT_ERR_DTYPE, "planar update: unsupported volume dtype");

@@ -334,7 +334,7 @@ def test_planar_sweep(ctx, nz, nviews, subset, order, style, du):
 @pytest.mark.parametrize("nrows,nsources", [(96, 1), (129, 1), (270, 1), (40, 3)])
 def test_objective_column_walk(ctx, nrows, nsources):
     """The objective of scans large enough for the column walk (2^25 ray and
-    plane pairs), rows in blocks of 128 and 256 with part blocks, and several
+    plane pairs and more), rows in blocks of 128 and 256 with part blocks, and several
     sources: the residual's 1e-5 bar on Ax doubled, as it enters squared and
     b = Ax/2 + 0.01."""
     g = Geometry(nx=64, ny=60, nz=52, vx=1.0, ncols=100, nrows=nrows, du=1.0, dv=90.0 / nrows, nviews=70,
@@ -345,6 +345,27 @@ def test_objective_column_walk(ctx, nrows, nsources):
     data, _, _ = ctx.objective(g, dev(x), dev(meas))
     want = float(((ref.astype(np.float64) - meas) ** 2).sum())
     assert abs(data - want) <= 4e-5 * want
+
+
+@pytest.mark.parametrize("nrows,subset", [(530, 1), (560, 2), (530, 3), (640, 5)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+def test_sweep_column_walk(ctx, nrows, subset, dt):
+    """Ray sums and sweeps of views large enough for the column walk (3 * 2^24
+    ray and plane pairs each), with rows in blocks of 128 and 256 and part
+    blocks: one view at a time, whose layout follows the direction, and
+    subsets of mixed directions on one layout or both.  Bars: 1e-5 on the
+    ray sums, 1e-4 on the reconstruction, 16-bit storage the rounding of one
+    stored update per subset."""
+    g = Geometry(nx=96, ny=92, nz=80, vx=1.0, ncols=512, nrows=nrows, du=0.33, dv=150.0 / nrows, nviews=5,
+                 angle_step_deg=37.0)
+    x = phantom(g, seed=2, scale=0.3).numpy()
+    x0 = (0.7 * x + 0.004).astype(np.float16).astype(np.float32)
+    b = orc.forward(g, x, prec=32)
+    v = dev(x0, dt)
+    assert rel(host(ctx.forward(g, v, out_dtype=torch.float32)), orc.forward(g, x0, prec=32)) <= 1e-5
+    ref = orc.sart_sweep(g, x0, b, beta=0.8, subset=subset, order="ascending", prec=32)
+    ctx.sart_sweep(g, v, dev(b), beta=0.8, subset=subset, order="ascending")
+    assert rel(host(v), ref) <= (1e-4 if dt == torch.float32 else 1e-3 * -(-5 // subset))
 
 
 @pytest.mark.parametrize("nz,nviews,kw", [(9, 1, {}), (9, 2, {}), (17, 67, {}), (7, 5, dict(nsources=3, src_z0=-4.0,
