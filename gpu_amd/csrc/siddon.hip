@@ -1604,12 +1604,13 @@ static bool adj_gather_fits(const DGeo<float> &d) {
 // rows on 420^3, 7/8 of the lanes, 11.2 -> 11.7 ms with 128; 560 on 280^3, 5/6,
 // 4.1 -> 4.0; FP16: 640 on 320^3, 5/6, 4.7 -> 4.4; gradient of 90 views of 96
 // rows on 64^3 217 -> 163 us).  Where 256 rows overrun the window, 128 serve;
-// not for corrections of FP32 volumes beyond the 32 MB of the XCDs' L2, nor on
-// 16-bit ones of fewer than four images or with more than an eighth of the lanes
-// past the last row: the per-ray walk is then the faster one (dv/vz = 1, FP32,
-// four views at a time: 200^3 0.82 -> 0.78 ms by column, 512^3 10.4 -> 11.3;
-// FP16: 512^3 10.2 -> 9.7, one at a time 4.4 -> 5.4; 420^3 with 504 rows
-// 5.5 -> 5.0, six at a time with 525 rows 8.5 -> 9.2).
+// not for corrections with more than an eighth of the lanes past the last row, of
+// FP32 volumes beyond the 32 MB of the XCDs' L2, or of fewer than four images on
+// 16-bit ones: the per-ray walk is then the faster one (dv/vz = 1, FP32, four
+// views at a time: 200^3 0.82 -> 0.78 ms by column, 512^3 10.4 -> 11.3; ten at a
+// time with 152 rows on 128^3 0.316 -> 0.329; FP16: 512^3 10.2 -> 9.7, one at a
+// time 4.4 -> 5.4; 420^3 with 504 rows 5.5 -> 5.0, six at a time with 525 rows
+// 8.5 -> 9.2).
 struct ColPlan { int rows, nq; };   // nq 0: the walk is not admitted
 static int col_quads(const DGeo<float> &d, int rw, int max_nq) {
     if ((d.ZP + rw - 1) / rw > 65535) return 0;
@@ -1652,8 +1653,8 @@ static ColPlan col_plan(const DGeo<float> &d, size_t es, int nimg, bool correcti
     const int n256 = q.n256, n128 = q.n128;
     const int pad256 = (d.ZP + 255) / 256 * 256, pad128 = (d.ZP + 127) / 128 * 128;
     if (n256 == 0) {
-        const bool ray = corrections && (es == 4 ? (uint64_t)d.M * d.N * d.Z * es > (32u << 20)
-                                                 : nimg < 4 || 8 * pad128 > 9 * d.ZP);
+        const bool ray = corrections && (8 * pad128 > 9 * d.ZP
+                                         || (es == 4 ? (uint64_t)d.M * d.N * d.Z * es > (32u << 20) : nimg < 4));
         return n128 > 0 && !ray ? ColPlan{128, n128} : none;
     }
     if (n128 > 0 && (es == 2 ? pad128 < pad256 : 4 * pad256 >= 5 * pad128)) return {128, n128};

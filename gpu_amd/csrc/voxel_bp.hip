@@ -350,8 +350,8 @@ __global__ __launch_bounds__(256) void k_bp_prep(DGeo<float> d, const float *__r
 }
 
 constexpr int BPX = 16, BPY = 16;
-// z-run per lane: 16 voxels for single-image launches, 8 when per-voxel sums
-// are carried across images (they live in registers)
+// longest z-run per lane: 16 voxels for single-image launches, 8 when per-voxel
+// sums are carried across images (they live in registers)
 template <bool ONE> constexpr int zrun() { return ONE ? 16 : 8; }
 constexpr int LW = 64;          // staged footprint columns
 constexpr int LP = LW + 8;      // LDS row pitch: 8 zero columns for the NC overrun
@@ -593,7 +593,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ONE ? 5 : 4
                                                       SV *__restrict__ f, const float2 *__restrict__ pixT,
                                                       const float4 *__restrict__ colT,
                                                       const float4 *__restrict__ rowT, int first, int stride,
-                                                      int nv, float beta, int mode) {
+                                                      int nv, float beta, int mode, int zr) {
     __shared__ float2 sp[LH * LP];   // (c*|S-P|, |S-P|); H: column-pair halves
     __shared__ float4 sc[LP];
     __shared__ float4 sr[LH];        // (qa, qb, 1/ez); H: (qa, qb, kl/ez)
@@ -603,8 +603,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ONE ? 5 : 4
     const int ix = tile.x * BPX + (TR ? threadIdx.y : threadIdx.x);
     const int iy = tile.y * BPY + (TR ? threadIdx.x : threadIdx.y);
     constexpr int ZR = zrun<ONE>();
-    const int iz0 = tile.z * ZR;
-    const int nz = min(ZR, d.Z - iz0);
+    const int iz0 = tile.z * zr;
+    const int nz = min(min(zr, ZR), d.Z - iz0);
     bool active = ix < d.M && iy < d.N;
     if (active) {   // cylinder mask
         const float hxm = (float)d.M * 0.5f - 0.5f, hym = (float)d.N * 0.5f - 0.5f;
@@ -1310,6 +1310,19 @@ static bool bp_lds_fits(const DGeo<float> &d, int zr) {
     return cols(DT) + 4.0 <= LW && rows(DT, zr * vz) + 4.0 <= LH && cols(DV) + 2.0 <= NCMAX;
 }
 
+// The z-run of a launch: the longest, halved while the chip is short of
+// workgroups (two per CU), where an update takes one run's latency.  A shorter run
+// repeats the tile's set-up and staging, so no further (sweeps, FP32: 32^3 / 50 x
+// 38, 8 single views 179 -> 123 us, 20 views in tens 180 -> 80; 96^3 / 154 x 114,
+// 20 views in tens 244 -> 174; 128^3 / 204 x 152, 8 views 254 -> 228, with four
+// workgroups per CU 242, with eight 274).
+static int bp_zrun(const DGeo<float> &d, int longest) {
+    const int64_t tiles = (int64_t)((d.M + BPX - 1) / BPX) * ((d.N + BPY - 1) / BPY);
+    int zr = longest;
+    while (zr > 1 && tiles * ((d.Z + zr - 1) / zr) < 512) zr >>= 1;
+    return zr;
+}
+
 // per-view tables, then the LDS-staged update (fast FP32 arithmetic)
 template <typename SV, bool ZQ, bool TR = false>
 static ct_status run_bp_lds(ct_context *ctx, const DGeo<float> &d, const float *ang, void *vol, const void *corr,
@@ -1330,16 +1343,16 @@ static ct_status run_bp_lds(ct_context *ctx, const DGeo<float> &d, const float *
     constexpr bool H = !std::is_same<SV, float>::value;
     hipLaunchKernelGGL(k_bp_prep<H>, dim3((d.R + 255) / 256, d.ZP, nimg), dim3(256), 0, ctx->stream, d, ang,
                        (const float *)corr, first, stride, pix, colT, rowT);
-    const int zr = nimg == 1 ? zrun<true>() : zrun<false>();
+    const int zr = bp_zrun(d, nimg == 1 ? zrun<true>() : zrun<false>());
     dim3 lgrid((d.M + BPX - 1) / BPX, (d.N + BPY - 1) / BPY, (d.Z + zr - 1) / zr);
     if (nimg == 1)
         hipLaunchKernelGGL((k_voxel_bp_lds<SV, true, H, ZQ, TR>), lgrid, dim3(BPX, BPY, 1), 0, ctx->stream, d, ang,
                            (SV *)vol, (const float2 *)pix, (const float4 *)colT, (const float4 *)rowT, first, stride,
-                           nv, (float)beta, mode);
+                           nv, (float)beta, mode, zr);
     else
         hipLaunchKernelGGL((k_voxel_bp_lds<SV, false, H, ZQ, TR>), lgrid, dim3(BPX, BPY, 1), 0, ctx->stream, d, ang,
                            (SV *)vol, (const float2 *)pix, (const float4 *)colT, (const float4 *)rowT, first, stride,
-                           nv, (float)beta, mode);
+                           nv, (float)beta, mode, zr);
     return launch_check(ctx, "voxel backprojection");
 }
 

@@ -368,6 +368,26 @@ def test_sweep_column_walk(ctx, nrows, subset, dt):
     assert rel(host(v), ref) <= (1e-4 if dt == torch.float32 else 1e-3 * -(-5 // subset))
 
 
+@pytest.mark.parametrize("n,nz", [(25, 1), (112, 43), (112, 90), (200, 37), (370, 17)])
+@pytest.mark.parametrize("subset", [1, 3])
+def test_sweep_z_runs(ctx, n, nz, subset):
+    """The staged update with runs of 16, 8, 4, 2 and 1 slices (volumes of few
+    and many tiles), each with a part run at the top, at the 1e-4
+    reconstruction bar against the FP32 oracle."""
+    # finer columns and rows than the magnified voxels, so that no voxel hangs
+    # on a single grazing ray; an odd grid with the odd detector's midline rays
+    rows = 2 * nz + 9
+    g = Geometry(nx=n | 1, ny=(n | 1) - 2, nz=nz | 1, vx=160.0 / n, ncols=2 * n + 1, nrows=rows, du=0.8 * 160.0 / n,
+                 nviews=4, angle_step_deg=37.3)
+    x = phantom(g, seed=2, scale=0.3).numpy()
+    b = orc.forward(g, x, prec=32)
+    x0 = 0.7 * x + 0.004
+    ref = orc.sart_sweep(g, x0, b, beta=0.8, subset=subset, order="ascending", prec=32)
+    v = dev(x0)
+    ctx.sart_sweep(g, v, dev(b), beta=0.8, subset=subset, order="ascending")
+    assert rel(host(v), ref) <= 1e-4
+
+
 @pytest.mark.parametrize("nz,nviews,kw", [(9, 1, {}), (9, 2, {}), (17, 67, {}), (7, 5, dict(nsources=3, src_z0=-4.0,
                                                                                             src_dz=4.0))])
 def test_adjoint_view_parts(ctx, nz, nviews, kw):
