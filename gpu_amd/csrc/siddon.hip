@@ -704,7 +704,7 @@ __global__ __launch_bounds__(RW) void k_project_col(DGeo<float> d, const float *
     unsigned *const ls = reinterpret_cast<unsigned *>(col_smem + 8 * LE); // x/y byte offset
     constexpr int ES = (int)sizeof(SV);
     const int tid = (int)threadIdx.x;
-    const int3 t = xcd_tile();
+    const int3 t = xcd_tile<true>();
     const int col = t.x, row0 = t.y * RW, row = row0 + tid;
     const int rowL = min(row0 + RW, d.ZP) - 1;
     const int img = t.z + z0;
