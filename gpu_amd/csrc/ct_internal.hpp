@@ -286,7 +286,7 @@ struct ProfScope {
 enum Slot {
     SLOT_CORR = 0,     // SART correction images
     SLOT_RED = 1,      // reduction partials
-    SLOT_FGP = 2,      // 9 FGP volumes (two dual sets, momentum copies)
+    SLOT_FGP = 2,      // 9 FGP volumes (three rotating sets of projected duals)
     SLOT_FDK = 3,      // weighted + filtered projection stack
     SLOT_TMP_VOL = 4,  // adjoint test / power iteration volumes
     SLOT_TMP_VOL2 = 5,
@@ -295,7 +295,7 @@ enum Slot {
     SLOT_FFT = 8,      // twiddles
     SLOT_MISC = 9,
     SLOT_BPTAB = 10,   // per-view tables of the fast voxel-driven backprojector
-    SLOT_ZQVOL = 11,   // the sweep's z-quad-layout volume
+    SLOT_ZQVOL = 11,   // the sweep's z-quad-layout volume (planar sweeps: z-fastest)
     SLOT_FDKV = 12,    // per-view constants of the fast FDK backprojector
     SLOT_IO = 13,      // FP32 staging of file reads and writes
     SLOT_ZQVOL_T = 14  // the sweep's volume in the transposed z-quad layout
