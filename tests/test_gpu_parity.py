@@ -405,6 +405,23 @@ def test_adjoint_view_parts(ctx, nz, nviews, kw):
     assert rel(got, ref) <= 2e-5
 
 
+@pytest.mark.parametrize("nx,ny,ncols", [(48, 48, 64), (46, 41, 60), (56, 56, 62)])
+def test_adjoint_truncated_detector(ctx, nx, ny, ncols):
+    """The gather adjoint of a volume wider than the detector, with coarse
+    voxels: voxels past the detector's last column lie in waves that still see
+    it, and read columns past the footprint.  A forward projection of NaNs goes
+    before, so that LDS that is read unwritten shows.  A 1.9 mm voxel spans
+    1.27e-3 of a ray's alpha, whose two crossings round to 6e-8 each: 9.4e-5
+    per segment at most, so 1e-4; against the FP32 oracle."""
+    stain = Geometry(nx=96, ny=92, nz=80, vx=1.0, ncols=512, nrows=530, du=0.33, dv=0.283, nviews=8)
+    ctx.forward(stain, torch.full(stain.vol_shape, float("nan"), device="cuda"))
+    g = Geometry(nx=nx, ny=ny, nz=13, vx=1.9, ncols=ncols, nrows=24, du=1.0, nviews=36)
+    y = np.random.default_rng(nx).standard_normal(g.proj_shape)
+    got = host(ctx.adjoint(g, dev(y)))
+    assert np.isfinite(got).all()
+    assert rel(got, orc.adjoint(g, y, prec=32)) <= 1e-4
+
+
 def test_adjoint_multisource_full_size(ctx):
     """The multi-source autograd geometry itself (48 sources 3 mm apart, 1024 x
     128 detector, 256^3 at 0.75 mm): the sources' spread needs 36 footprint
