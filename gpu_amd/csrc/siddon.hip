@@ -1308,6 +1308,7 @@ __device__ __forceinline__ float adj_rows(const float *__restrict__ sw, const fl
                                           const float2 *__restrict__ srl, int z0, int z1, int cbase, float n, float n1,
                                           const float *xin, const float *xout) {
     float acc = 0.0f;
+    if (z1 < z0) return acc;   // (a slice past the volume or the staged rows: no pointer to form)
     const float *prow = sw + (__umul24((uint32_t)z0, ALP) + cbase);
     const float2 *lp = srl + z0;
     for (const float2 *rp = srk + z0, *const re = srk + z1; rp <= re; ++rp, prow += ALP) {
