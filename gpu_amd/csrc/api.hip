@@ -48,6 +48,19 @@ void *slot(ct_context *ctx, int which, size_t bytes, ct_status *st) {
     return p;
 }
 
+void *slot_or_null(ct_context *ctx, int which, size_t bytes) {
+    if (ctx->slots[which].bytes < bytes && ctx->stream) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess) hipGetLastError();
+        if (cs != hipStreamCaptureStatusNone) return nullptr;
+    }
+    const std::string was = ctx->last_error;
+    ct_status st;
+    void *p = slot(ctx, which, bytes, &st);
+    if (!p) ctx->last_error = was;
+    return p;
+}
+
 // Per-view angles exactly as the reference host code forms them
 // (V63/host_IterativeRecon_CBCT.c:34-41, FDK: V63/host_FDK.cpp:35-40).
 template <typename T> static void angle_host(const ct_geometry &g, int j, bool fdk, T &s, T &c) {
@@ -224,11 +237,10 @@ static ct_status sweep(ct_context *ctx, const ct_geometry &g, void *vol, ct_dtyp
         if (tr && (st = launch_zq_transpose(ctx, volt, vdt, volq, g.nx, g.ny, g.nz, false)) != CT_OK) return st;
         return launch_zq_unpack(ctx, volq, vdt, vol, g.nx, g.ny, g.nz);
     }
-    if (planar_sweep_fits(ctx, g, vdt, subset)) {
+    void *volz = planar_sweep_fits(ctx, g, vdt, subset) ? planar_sweep_scratch(ctx, g, vdt) : nullptr;
+    if (volz) {
         // fan and parallel beam with the rows at the slice centres: the sweep
         // runs on a z-fastest copy of the volume
-        void *volz = slot(ctx, SLOT_ZQVOL, (size_t)vox(&g) * dtype_size(vdt), &st);
-        if (!volz) return st;
         if ((st = launch_zfast(ctx, vol, vdt, volz, g.nx, g.ny, g.nz, true)) != CT_OK) return st;
         auto step = [&](int first, int stride, int cnt) {
             ct_status s2 = launch_planar_corr(ctx, g, volz, vdt, (float *)corr, meas, mdt, first, stride, cnt);

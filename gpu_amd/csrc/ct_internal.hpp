@@ -305,6 +305,10 @@ ct_status fail(ct_context *ctx, ct_status s, const std::string &msg);
 ct_status hip_check(ct_context *ctx, hipError_t e, const char *what);
 ct_status launch_check(ct_context *ctx, const char *what);
 void *slot(ct_context *ctx, int which, size_t bytes, ct_status *st);
+// A slot that the call can do without (a copy of the volume that makes it
+// faster): null, and no error left, where the memory is not there or where the
+// slot would have to grow while the stream is captured into a graph.
+void *slot_or_null(ct_context *ctx, int which, size_t bytes);
 // Device angle table (T = float or double), sin at [2v], cos at [2v+1].
 const void *angle_table(ct_context *ctx, const ct_geometry &g, bool dbl, bool fdk, ct_status *st);
 // the same table in host memory (g.nviews (sin, cos) pairs, float or double)
@@ -359,6 +363,8 @@ ct_status launch_voxel_bp_zq(ct_context *ctx, const ct_geometry &g, void *volq, 
 // Planar sweep (fan or parallel beam with the rows at the slice centres): the
 // volume in the z-fastest layout [y][x][z], corrections [image][column][row]
 bool planar_sweep_fits(const ct_context *ctx, const ct_geometry &g, ct_dtype vdt, int subset);
+// its scratch: the z-fastest volume; null where the general path has to serve
+void *planar_sweep_scratch(ct_context *ctx, const ct_geometry &g, ct_dtype vdt);
 ct_status launch_zfast(ct_context *ctx, const void *in, ct_dtype dt, void *out, int M, int N, int Z, bool to_zfast);
 ct_status launch_planar_corr(ct_context *ctx, const ct_geometry &g, const void *volz, ct_dtype vdt, float *corr,
                              const void *meas, ct_dtype mdt, int32_t first, int32_t stride, int32_t nv);

@@ -1776,9 +1776,12 @@ static ct_status launch_col(ct_context *ctx, const ct_geometry &g, const DGeo<fl
     // (FP32, 263 x 261 x 251 / 549 x 459, three views and two: 0.19 ms, 0.23 on
     // the layout that is there; 512^3 / 1024^2 in subsets of four 22.4 ms, 23.0
     // with the copy).  So do all of a BF16 sweep's, at all sizes (sweep_plan).
+    // And so does any launch for which there is no memory for the other copy.
     const bool few = others * d.NS < 4 || (CMD == 1 && std::is_same<SV, __hip_bfloat16>::value);
+    const uint64_t bytes = (uint64_t)d.M * d.N * (uint64_t)((d.Z + 3) & ~3) * sizeof(SV);
+    void *t = few ? nullptr : slot_or_null(ctx, tr ? SLOT_ZQVOL : SLOT_ZQVOL_T, bytes);
     if constexpr (CMD != 2) {
-        if (others > 0 && few && !tr) {
+        if (others > 0 && !t && !tr) {
             const int64_t P = (int64_t)d.R * d.ZP * d.NS;
             for (int q0 = 0, q1; q0 < nv; q0 = q1) {
                 const bool w = col_walk_view(g, first + q0 * stride);
@@ -1790,12 +1793,8 @@ static ct_status launch_col(ct_context *ctx, const ct_geometry &g, const DGeo<fl
             return CT_OK;
         }
     }
-    if (!few) {
-        ct_status st;
-        const uint64_t bytes = (uint64_t)d.M * d.N * (uint64_t)((d.Z + 3) & ~3) * sizeof(SV);
-        void *t = slot(ctx, tr ? SLOT_ZQVOL : SLOT_ZQVOL_T, bytes, &st);
-        if (!t) return st;
-        st = launch_zq_transpose(ctx, volq, dtype_of<SV>(), t, d.M, d.N, d.Z, !tr);
+    if (t) {
+        const ct_status st = launch_zq_transpose(ctx, volq, dtype_of<SV>(), t, d.M, d.N, d.Z, !tr);
         if (st != CT_OK) return st;
         vols[!tr] = t;
     }
@@ -1814,16 +1813,15 @@ static ct_status run_residual(ct_context *ctx, const ct_geometry &g, const void 
     const bool comp = std::is_same<T, float>::value && ctx->math == CT_MATH_FAST;
     if constexpr (std::is_same<T, float>::value) {
         // the batched ray sums' column walk where it outweighs the copies of
-        // the volume
+        // the volume, and there is memory for one
         const uint64_t qbytes = (uint64_t)d.M * d.N * (uint64_t)((d.Z + 3) & ~3) * sizeof(SV);
         const bool large = col_pairs(d, nimg) >= 2 * COL_MIN;
         const ColPlan cp = comp && large && nimg >= 4 && qbytes < (1ull << 32) ? col_plan(d, sizeof(SV), nimg, false) : ColPlan{0, 0};
-        if (cp.nq > 0) {
+        void *volq = cp.nq > 0 ? slot_or_null(ctx, SLOT_ZQVOL, qbytes) : nullptr;
+        if (volq) {
             const int64_t per = (int64_t)d.R * ((d.ZP + cp.rows - 1) / cp.rows);   // workgroups per image
             double *part = (double *)slot(ctx, SLOT_TMP_PROJ2, sizeof(double) * per * nimg, &st);
             if (!part) return st;
-            void *volq = slot(ctx, SLOT_ZQVOL, qbytes, &st);
-            if (!volq) return st;
             {
                 ProfScope ps(ctx, CT_K_FORWARD);
                 st = launch_zq_pack(ctx, vol, dtype_of<SV>(), volq, d.M, d.N, d.Z);
@@ -2234,13 +2232,17 @@ static ct_status run_adjoint_gather(ct_context *ctx, const ct_geometry &g, const
     if (!ang) return st;
     const int nimg = nv * d.NS;
     const size_t P = (size_t)d.R * d.ZP;
-    const int parts = adj_parts(d, nv);
+    int parts = adj_parts(d, nv);
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t pw_b = up(sizeof(float) * P * nimg), col_b = up(sizeof(AdjCol) * (size_t)d.R * nv);
     const size_t row_b = up(sizeof(float4) * (size_t)d.ZP * nimg);
     const size_t part_b = parts > 1 ? sizeof(float2) * (size_t)d.M * d.N * d.Z * parts : 0;
-    char *tab = (char *)slot(ctx, SLOT_TMP_VOL, pw_b + col_b + row_b + part_b, &st);
-    if (!tab) return st;
+    char *tab = parts > 1 ? (char *)slot_or_null(ctx, SLOT_TMP_VOL, pw_b + col_b + row_b + part_b) : nullptr;
+    if (!tab) {   // in one part if it has to be
+        parts = 1;
+        tab = (char *)slot(ctx, SLOT_TMP_VOL, pw_b + col_b + row_b, &st);
+        if (!tab) return st;
+    }
     float *pixw = (float *)tab;
     AdjCol *colT = (AdjCol *)(tab + pw_b);
     float4 *rowT = (float4 *)(tab + pw_b + col_b);

@@ -1237,6 +1237,13 @@ bool planar_sweep_fits(const ct_context *ctx, const ct_geometry &g, ct_dtype vdt
     return ((1.0 + rmax) * DV + dr * DV * lat) / (double)d.du + 2.0 <= PMAXC;
 }
 
+// bytes of a view's chords and words
+static size_t planar_table_bytes(int M, int N) { return (size_t)M * N * (PMAXC * sizeof(float) + sizeof(int)); }
+void *planar_sweep_scratch(ct_context *ctx, const ct_geometry &g, ct_dtype vdt) {
+    if (!slot_or_null(ctx, SLOT_BPTAB, planar_table_bytes(g.nx, g.ny))) return nullptr;
+    return slot_or_null(ctx, SLOT_ZQVOL, (size_t)g.nx * g.ny * g.nz * dtype_size(vdt));
+}
+
 template <typename SV>
 static ct_status planar_update(ct_context *ctx, const DGeo<float> &d, const float *ang, void *volz, const float *corr,
                                int first, int stride, int nv, double beta) {
@@ -1248,7 +1255,7 @@ static ct_status planar_update(ct_context *ctx, const DGeo<float> &d, const floa
     }
     ct_status st;
     const size_t cells = (size_t)d.M * d.N;
-    float *lens = (float *)slot(ctx, SLOT_BPTAB, cells * (PMAXC * sizeof(float) + sizeof(int)), &st);
+    float *lens = (float *)slot(ctx, SLOT_BPTAB, planar_table_bytes(d.M, d.N), &st);
     if (!lens) return st;
     int *word = (int *)(lens + cells * PMAXC);
     hipLaunchKernelGGL(k_planar_chords, dim3((d.M + 63) / 64, (d.N + 3) / 4), dim3(256), 0, ctx->stream, d, ang, first,
