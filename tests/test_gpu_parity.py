@@ -388,6 +388,26 @@ def test_sweep_z_runs(ctx, n, nz, subset):
     assert rel(host(v), ref) <= 1e-4
 
 
+@pytest.mark.parametrize("nz,run", [(301, 2), (201, 1)])
+@pytest.mark.parametrize("subset", [1, 3])
+def test_sweep_short_z_runs(ctx, nz, run, subset):
+    """The staged update with the runs of 2 and 1 slices of narrow volumes, whose
+    tiles are four: a run is halved while that gives fewer than 512 workgroups.
+    The 1e-4 reconstruction bar against the FP32 oracle."""
+    zr = 8 if subset > 1 else 16
+    while zr > 1 and 4 * -(-nz // zr) < 512:
+        zr //= 2
+    assert zr == run
+    g = Geometry(nx=25, ny=23, nz=nz, vx=1.0, ncols=51, nrows=2 * nz + 9, du=0.8, nviews=4, angle_step_deg=37.3)
+    x = phantom(g, seed=2, scale=0.3).numpy()
+    b = orc.forward(g, x, prec=32)
+    x0 = 0.7 * x + 0.004
+    ref = orc.sart_sweep(g, x0, b, beta=0.8, subset=subset, order="ascending", prec=32)
+    v = dev(x0)
+    ctx.sart_sweep(g, v, dev(b), beta=0.8, subset=subset, order="ascending")
+    assert rel(host(v), ref) <= 1e-4
+
+
 @pytest.mark.parametrize("nz,nviews,kw", [(9, 1, {}), (9, 2, {}), (17, 67, {}), (7, 5, dict(nsources=3, src_z0=-4.0,
                                                                                             src_dz=4.0))])
 def test_adjoint_view_parts(ctx, nz, nviews, kw):
