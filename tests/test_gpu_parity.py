@@ -763,6 +763,19 @@ def test_tv_fgp_tile_edges(ctx, shape, niter):
     assert float(np.abs(host(h) - ref).max()) <= 2.0 ** -11 + 0.004 * 12 * 2.0 ** -11 * (1 + niter)
 
 
+def test_tv_fgp_tall_strips(ctx):
+    """The strips of 8 rows that FP32 volumes of 2^25 voxels and more take, with
+    a remainder in x, y and z: bit-identical to the oracle."""
+    shape = (327, 325, 323)
+    assert math.prod(shape) >= 1 << 25
+    b = np.random.default_rng(12).random(shape, dtype=np.float32)
+    ref = orc.tv_fgp(b, 0.004, 3, prec=32)
+    v = dev(b)
+    ctx.tv_fgp(v, 0.004, 3)
+    torch.cuda.synchronize()
+    assert np.array_equal(v.cpu().numpy(), ref)
+
+
 @pytest.mark.parametrize("ncols", [1, 3, 129, 255, 257, 513, 720, 1025, 2047])
 def test_ramp_filter_transform_lengths(ctx, ncols):
     """Row lengths around the transform lengths 2^9..2^12, whose taps' spectrum
