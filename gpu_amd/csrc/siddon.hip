@@ -1446,10 +1446,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         const int y1r = shadow_hi((maxY - d.ymin) * d.idu);
         const int y0 = max(y0r, C0), y1 = min(min(y1r, C1), y0 + ANC - 1);
         // (a lane off the volume or the detector has no columns; it still reads
-        // its wave's NC, so they start at ncw at the latest: of the staged rows
-        // only the footprint and the eight zero columns after it are written)
+        // its wave's NC, and takes them from ncw on: of the staged rows only the
+        // footprint and the eight zero columns after it are written, and a
+        // pixel that is not finite must not reach it, not even times 0)
         const int ncol = active ? max(y1 - y0 + 1, 0) : 0;
-        const int cbase = min(max(y0 - C0, 0), ncw);
+        const int cbase = ncol > 0 ? y0 - C0 : ncw;
         int NC = 0;   // uniform over the wave
         bool fresh = true;
         float xin[ANC], xout[ANC];

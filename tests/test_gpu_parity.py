@@ -459,6 +459,26 @@ def test_adjoint_slices_without_rows(ctx, nz, nrows, src_z0):
     assert len(far) > 0 and not np.any(got[far])
 
 
+@pytest.mark.parametrize("ncols,off", [(4, 0.0), (7, -3.0), (7, 3.0)])
+@pytest.mark.parametrize("val", [math.inf, math.nan])
+def test_adjoint_nonfinite_pixel(ctx, ncols, off, val):
+    """A pixel that is not finite leaves the voxels whose corners all project
+    beside the detector alone, left and right of it: exactly zero from one view."""
+    g = small_geom(nx=30, ny=18, nz=13, ncols=ncols, nrows=25, det_offset=off, nviews=1, angle0_deg=20.0)
+    y = np.ones(g.proj_shape)
+    y[0, :, 0] = y[0, :, -1] = val
+    got = host(ctx.adjoint(g, dev(y)))
+    s, c = core.view_angle(g, 0)
+    X, Y = np.meshgrid(np.arange(g.nx + 1) - g.nx / 2, np.arange(g.ny + 1) - g.ny / 2)
+    t, sv = X * c + Y * s, -X * s + Y * c
+    u = (t - g.dod) / (g.dso - t) * (sv - off) + sv
+    corners = [u[a:a + g.ny, b:b + g.nx] for a in (0, 1) for b in (0, 1)]
+    first = off - g.du * (ncols - 1) / 2
+    beside = (np.max(corners, axis=0) < first - 0.05) | (np.min(corners, axis=0) > first + g.du * (ncols - 1) + 0.05)
+    assert beside.any() and not np.any(got[:, beside])
+    assert not np.isfinite(got).all()
+
+
 def test_adjoint_multisource_full_size(ctx):
     """The multi-source autograd geometry itself (48 sources 3 mm apart, 1024 x
     128 detector, 256^3 at 0.75 mm): the sources' spread needs 36 footprint
