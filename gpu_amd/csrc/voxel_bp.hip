@@ -1099,8 +1099,9 @@ __global__ __launch_bounds__(256) void k_planar_one(DGeo<float> d, SV *__restric
     typename RawOf<SV>::type xr[PONE];
     float cv[PONE][PC];
     int w[PONE];
-    // (columns past a cell's own repeat its last one with length 0; a cell
-    // without chords, masked ones among them, is not touched)
+    // (columns past a cell's own repeat its last one, and the sums stop before
+    // them: a correction that is not finite counts once; a cell without chords,
+    // masked ones among them, is not touched)
 #pragma unroll
     for (int n = 0; n < PONE; ++n) {
         w[n] = c0 + n < MN ? word[c0 + n] : 0;
@@ -1118,9 +1119,9 @@ __global__ __launch_bounds__(256) void k_planar_one(DGeo<float> d, SV *__restric
         float wk = 0.0f, lk = 0.0f;
 #pragma unroll
         for (int k = 0; k < PC; ++k) {
-            const float l = k < cnt ? len[k] : 0.0f;
-            lk += l;
-            wk = fmaf(l, cv[n][k], wk);
+            if (k >= cnt) break;   // uniform
+            lk += len[k];
+            wk = fmaf(len[k], cv[n][k], wk);
         }
         for (int k = PC; k < cnt; ++k) {
             lk += len[k];
@@ -1156,7 +1157,7 @@ __global__ __launch_bounds__(256) void k_planar_many(DGeo<float> d, const float 
         __syncthreads();
         if (z >= d.Z) continue;
         // PB cells at a time, so that their correction loads are in flight
-        // together; columns past a cell's own repeat its last one with length 0
+        // together; columns past a cell's own repeat its last one, unused
         constexpr int PB = 4, PC = 4;
 #pragma unroll
         for (int n0 = 0; n0 < PCELL; n0 += PB) {
@@ -1182,7 +1183,8 @@ __global__ __launch_bounds__(256) void k_planar_many(DGeo<float> d, const float 
                     float wk = W[n0 + n], lk = L[n0 + n];
 #pragma unroll
                     for (int k = 0; k < PC; ++k) {
-                        const float len = k < cnt ? slen[q][cl][ca + k] : 0.0f;
+                        if (k >= cnt) break;   // uniform
+                        const float len = slen[q][cl][ca + k];
                         lk += len;
                         wk = fmaf(len, cv[n][k], wk);
                     }

@@ -331,6 +331,31 @@ def test_planar_sweep(ctx, nz, nviews, subset, order, style, du):
     assert rel(host(h), ref) <= 1e-3 * -(-nviews // subset)
 
 
+@pytest.mark.parametrize("style", [1, 2])
+@pytest.mark.parametrize("views", [1, 3])
+@pytest.mark.parametrize("what,val", [("meas", math.inf), ("meas", -math.inf), ("meas", math.nan), ("vol", -math.inf)])
+def test_planar_sweep_nonfinite(ctx, style, views, what, val):
+    """One update of a fan or parallel sweep with a pixel or a voxel that is not
+    finite: infinities and NaNs reach the voxels they reach in the reference, and
+    no other."""
+    g = small_geom(nx=21, ny=26, nz=13, nrows=13, dv=1.0, ncols=37, du=0.9, nviews=views, style=style,
+                   angle0_deg=20.0)
+    x = phantom(g, seed=2, scale=0.3).numpy()
+    b = orc.forward(g, x, prec=32)
+    x0 = (0.7 * x + 0.004).astype(np.float32)
+    (b if what == "meas" else x0)[(0, 6, 17) if what == "meas" else (6, 14, 9)] = val
+    ref = orc.sart_sweep(g, x0, b, beta=0.8, subset=views, order="ascending", prec=32)
+    v = dev(x0)
+    ctx.sart_sweep(g, v, dev(b), beta=0.8, subset=views)
+    got = host(v)
+    assert not np.isfinite(ref).all()
+    ok = np.isfinite(ref)
+    assert np.array_equal(np.isfinite(got), ok)
+    # (the compensated ray sums of fast mode turn an infinite voxel into NaN)
+    assert what == "vol" or np.array_equal(np.isnan(got), np.isnan(ref))
+    assert rel(got[ok], ref[ok]) <= 1e-4
+
+
 @pytest.mark.parametrize("nrows,nsources", [(96, 1), (129, 1), (270, 1), (40, 3)])
 def test_objective_column_walk(ctx, nrows, nsources):
     """The objective of scans large enough for the column walk (2^25 ray and
