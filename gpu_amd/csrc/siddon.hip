@@ -826,7 +826,14 @@ __global__ __launch_bounds__(RW) void k_project_col(DGeo<float> d, const float *
     int zrb = 0, dzb = 0;
     if (!cmiss && row < d.ZP && fw.init(d, s, c, col, row, src)) {
         len = fw.len; dist = fw.dist;
-        if constexpr (CMD != 1) {
+        if constexpr (CMD == 1) {
+            // a level ray (kz = 0) keeps the slab the walk puts it in, which
+            // the rounding of zeta would decide where it lies in a slice plane
+            if (fw.kz == 0.0f) {
+                cz = 0.0f; icz = 0.0f;
+                z0c = fw.nfz - (fw.sgzf > 0.0f ? 1.0f : 0.0f) - (float)(kbb / SB) + 0.5f;
+            }
+        } else {
             lo = fw.ac; hi = fw.amax;
             az = fw.az; nfz = fw.nfz; kz = fw.kz; bz0 = fw.bz0; sgzf = fw.sgzf;
             zrb = ((int)nfz - (sgzf > 0.0f ? 1 : 0)) * SB - kbb;

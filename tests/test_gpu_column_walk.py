@@ -105,3 +105,15 @@ def test_row_blocks(dt, nrows):
 @pytest.mark.parametrize("dt", DTYPES)
 def test_geometries(dt, kw):
     check(replace(SMALL, **kw), dt, 11)
+
+
+@pytest.mark.parametrize("kw", [
+    dict(nz=6, vz=0.7, ncols=11, nrows=17, dv=1.1146163743152828, nsources=5, src_z0=-12.0, src_dz=6.0),
+    dict(nz=58, vz=0.35, ncols=21, nrows=41, dv=0.30271779082383904),
+], ids=["five sources", "one source"])
+@pytest.mark.parametrize("dt", DTYPES)
+def test_level_rays(dt, kw):
+    """A middle row that lies level with a source, to rounding in the plane
+    between two slices: the whole row belongs to the slab that the reference's
+    set-up puts it in."""
+    check(replace(SMALL, **kw), dt, 5)
