@@ -418,14 +418,30 @@ template <int ES, bool ZQ = false> struct FastWalk {
         ac = m;
         return dl;
     }
+    // z planes counted from the multiple of four next to the first crossing,
+    // whose alpha has no cancellation left: on nearly level rays, where a plane
+    // spans much alpha, the rounding of plane 0's would move every crossing.
+    // Returns that plane (restart takes it).
+    __device__ __forceinline__ int rebase_z(const DGeo<float> &d, float s, float c, int col, int row, int src) {
+        if (kz == 0.0f) return 0;
+        const float z1 = d.zmin + (float)row * d.dv;
+        float sx, sy, z2;
+        ray_source(d, s, c, d.ymin + (float)col * d.du, z1, src, sx, sy, z2);
+        const float n0 = 4.0f * floorf(nfz * 0.25f);
+        bz0 = (fmaf(n0, d.vz, d.bz) - z1) / (z2 - z1);
+        nfz -= n0;
+        az = fmaf(nfz, kz, bz0);
+        return (int)n0;
+    }
     __device__ __forceinline__ bool ended() const { return !(amax - ac > loop_eps<float>()); }
     // continue the walk from alpha a in [ac, amax]: the slab of each
     // stepping axis that holds a (as start() finds it), its pending crossing
     // and the voxel offset
-    __device__ __forceinline__ void restart(const DGeo<float> &d, float a) {
+    // (zq: the plane index that nfz and bz0 count from, see rebase_z)
+    __device__ __forceinline__ void restart(const DGeo<float> &d, float a, int zq = 0) {
         const int vi = restart_axis(kx, bx0, sgxf, nfx, a, d.M);
         const int vj = restart_axis(ky, by0, sgyf, nfy, a, d.N);
-        const int vk = restart_axis(kz, bz0, sgzf, nfz, a, d.Z);
+        const int vk = restart_axis(kz, bz0, sgzf, nfz, a, d.Z - zq, -zq) + zq;
         ax = fmaf(nfx, kx, bx0); ay = fmaf(nfy, ky, by0); az = fmaf(nfz, kz, bz0);
         const unsigned M = d.M, MN = (unsigned)d.M * (unsigned)d.N;
         if constexpr (ZQ)
@@ -434,14 +450,14 @@ template <int ES, bool ZQ = false> struct FastWalk {
             idx = ((unsigned)vk * MN + (unsigned)vj * M + (unsigned)vi) * (unsigned)ES;
         ac = a;
     }
-    __device__ __forceinline__ static int restart_axis(float k, float b0, float sg, float &nf, float a, int n) {
+    __device__ __forceinline__ static int restart_axis(float k, float b0, float sg, float &nf, float a, int n, int first = 0) {
         const int up = sg > 0.0f;
         if (k == 0.0f) return (int)nf - up;   // parallel axis: its slab never changes
         const int sgi = up ? 1 : -1;
-        int v = min(max((int)floorf((a - b0) / k), 0), n - 1);
+        int v = min(max((int)floorf((a - b0) / k), first), n - 1);
         if (fmaf((float)(v + 1 - up), k, b0) > a) v -= sgi;     // a lies before the entry plane
         else if (fmaf((float)(v + up), k, b0) < a) v += sgi;    // a lies past the exit plane
-        v = min(max(v, 0), n - 1);
+        v = min(max(v, first), n - 1);
         nf = (float)(v + up);
         return v;
     }
@@ -592,9 +608,13 @@ __global__ __launch_bounds__(256) void k_project_zq(DGeo<float> d, const float *
             len = fw.len;
             dist = fw.dist;
             if constexpr (S > 1) {
+                // (16-bit volumes, whose storage rounding hides it and whose
+                // stored updates are dithered from the sums' low bits, do without)
+                int zq = 0;
+                if constexpr (std::is_same<SV, float>::value) zq = fw.rebase_z(d, s, c, col, row, src);
                 const float lo = fw.ac, span = fw.amax - fw.ac;
                 if (p + 1 < S) fw.amax = fmaf(span, (float)(p + 1) / (float)S, lo);
-                if (p > 0) fw.restart(d, fmaf(span, (float)p / (float)S, lo));
+                if (p > 0) fw.restart(d, fmaf(span, (float)p / (float)S, lo), zq);
             }
             sum = walk_sum<SV, true, true>(fw, d, fq);
         }
