@@ -112,8 +112,8 @@ __device__ __forceinline__ float hmin3(float a, float b, float c) {
 // takes ANY (objective of 292 x 312 x 277, FP32, 35 views of 554 columns, 38780
 // workgroups: 3.73 ms round-robin, 1.97 contiguous); the kernels that work by
 // volume tile don't, whose eighths carry unequal work where the detector does
-// not reach the end slices (gradient of 264 x 290 x 267 from 82 rows 0.84 ms
-// round-robin, 1.87 contiguous; FDK of 389 x 419 x 337 3.95 and 4.06).
+// not reach the end slices (FDK of 389 x 419 x 337 3.95 ms round-robin, 4.06
+// contiguous; the gather adjoint has an order of its own, xcd_rows).
 template <bool ANY = false> __device__ __forceinline__ int3 xcd_tile() {
     const unsigned gx = gridDim.x, gy = gridDim.y, T = gx * gy * gridDim.z;
     const unsigned L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);

@@ -529,9 +529,12 @@ __device__ __forceinline__ double lane_value(double v, int l) { return __shfl(v,
 // The waves of a workgroup lie side by side in x (2^lx of them, the rest
 // stacked in y), so that it touches whole rows of up to 1 KiB: with the waves
 // stacked in y instead the pass takes 1.25 ms at 512^3 in FP32, side by side
-// 1.04 (4.9 TB/s over its 10 words; a large copy runs at 4.6), against 1.38
-// for the form with LDS staging and the momentum point in memory.  FP16 on 500
-// x 468 x 391: 0.87 -> 0.55 ms.
+// 1.06 on the mean of 20, against 1.38 for the form with LDS staging and the
+// momentum point in memory.  Bound by HBM: a pass with both sets moves 6.5 GB in
+// 1.11 ms, 5.8 TB/s, 1.21 times its 10 words per voxel for the rows above and
+// below a wave's.  FP16 on 500 x 468 x 391: 0.87 -> 0.55 ms on the mean; a pass
+// with both sets moves 3.3 GB in 0.61 ms, 5.5 TB/s, but 1.8 times its 10 words,
+// as strips of 4 rows read 6.
 constexpr int FGW = 4;                       // waves per workgroup
 
 template <typename S, typename T, typename D, int FIRST, int FGR>

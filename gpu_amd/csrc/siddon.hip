@@ -1054,8 +1054,9 @@ __global__ __launch_bounds__(RW) void k_project_col(DGeo<float> d, const float *
 // Kahan-compensated, as in the other walks.  The corrections are stored
 // [image][column][row], as k_planar_update reads them.
 //
-// Bound by L2: 512 x 512 x 256 / 1024 x 256 0.052 ms per view, against 0.28 ms
-// for one per-ray walk per lane.
+// Bound by memory, the volume read once: 512 x 512 x 256 / 1024 x 256 0.055 ms
+// and 272 MB of HBM per view (5.0 TB/s; VALU issue 27%), against 0.28 ms for one
+// per-ray walk per lane.
 template <typename SV, typename SM>
 __global__ __launch_bounds__(256) void k_planar_corr(DGeo<float> d, const float *__restrict__ ang,
                                                      const SV *__restrict__ fz, float *__restrict__ corr,
@@ -1359,6 +1360,22 @@ __device__ __forceinline__ float adj_rows(const float *__restrict__ sw, const fl
     return acc;
 }
 
+// The gather's tiles: two rows of tiles to each XCD in turn.  Whole eighths of
+// the volume (xcd_tile) leave the XCDs of the end slices idle where the detector
+// does not reach them, single tiles share no lines of the tables (gradient of many
+// sources in BF16 4.43 ms by eighths, 2.60 by tile, 2.53, 2.49 and
+// 2.53 by one, two and four rows; 512^3 / 1024^2, 24 views 12.3, 12.6, 12.3,
+// 12.0, 12.0).  The rest past a multiple of eight such chunks keeps its order.
+__device__ __forceinline__ int3 xcd_rows() {
+    const unsigned gx = gridDim.x, gy = gridDim.y, T = gx * gy * gridDim.z, C = gx * 2;
+    const unsigned L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
+    const unsigned i = L >> 3, q = i / C;
+    const unsigned t = (q + 1) * 8 * C <= T ? (q * 8 + (L & 7u)) * C + (i - q * C) : L;
+    const unsigned z = t / (gx * gy), r = t - z * (gx * gy);
+    const unsigned y = r / gx;
+    return make_int3((int)(r - y * gx), (int)y, (int)z);
+}
+
 // one lane per (x, y) and its AZR z-voxels; a 16x16 (x, y) tile per
 // workgroup; per image the tile's detector footprint of weights is staged in
 // LDS.  Each image's per-voxel sum (FP32, ~10 terms) is added into an FP32
@@ -1378,22 +1395,6 @@ __device__ __forceinline__ float adj_rows(const float *__restrict__ sw, const fl
 // volumes whose tiles leave the chip idle; part p's sums and their
 // compensations go to part[p V + voxel] and k_adj_fold adds them in FP64.
 // 64^3 from 90 views of 96^2: 730 us on its 128 tiles, 80 us in 1024 parts.
-// The gather's tiles: two rows of tiles to each XCD in turn.  Whole eighths of
-// the volume (xcd_tile) leave the XCDs of the end slices idle where the detector
-// does not reach them, single tiles share no lines of the tables (gradient of many
-// sources in BF16 4.43 ms by eighths, 2.60 by tile, 2.53, 2.49 and
-// 2.53 by one, two and four rows; 512^3 / 1024^2, 24 views 12.3, 12.6, 12.3,
-// 12.0, 12.0).  The rest past a multiple of eight such chunks keeps its order.
-__device__ __forceinline__ int3 xcd_rows() {
-    const unsigned gx = gridDim.x, gy = gridDim.y, T = gx * gy * gridDim.z, C = gx * 2;
-    const unsigned L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-    const unsigned i = L >> 3, q = i / C;
-    const unsigned t = (q + 1) * 8 * C <= T ? (q * 8 + (L & 7u)) * C + (i - q * C) : L;
-    const unsigned z = t / (gx * gy), r = t - z * (gx * gy);
-    const unsigned y = r / gx;
-    return make_int3((int)(r - y * gx), (int)y, (int)z);
-}
-
 template <typename SO, bool PART>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_adjoint_gather(DGeo<float> d, const float *__restrict__ ang, int view0,
                                                         int nv, int vpp, const float *__restrict__ pixw,

@@ -1011,10 +1011,12 @@ static bool planar_eligible(const ct_context *ctx, const DGeo<float> &d) {
 //
 // One view: k_planar_chords lists the chords of all cells, and k_planar_one
 // streams the volume, eight cells per lane in flight.  Bound by memory (the
-// volume read and written): 512 x 512 x 256 0.124 ms per view in FP32, the
-// chords included, against 0.20 ms with the chords formed in the same kernel
-// (every workgroup waits for its few chord threads) and 0.23 ms with a lane
-// per (x, y) and 16 slices, whose corrections were one gather per slice.
+// volume read and written): 512 x 512 x 256 0.114 ms per view in FP32, the
+// chords included (440 MB of HBM in 0.106 ms, VALU issue 24%; 0.124 ms before
+// the products past a cell's columns were branched around), against 0.20 ms with
+// the chords formed in the same kernel (every workgroup waits for its few chord
+// threads) and 0.23 ms with a lane per (x, y) and 16 slices, whose corrections
+// were one gather per slice.
 //
 // Several views: k_planar_many takes PVIEW views at a time into LDS and keeps
 // its cells' sums in registers, so the volume is read and written once.
