@@ -531,10 +531,11 @@ __device__ __forceinline__ double lane_value(double v, int l) { return __shfl(v,
 // stacked in y instead the pass takes 1.25 ms at 512^3 in FP32, side by side
 // 1.06 on the mean of 20, against 1.38 for the form with LDS staging and the
 // momentum point in memory.  Bound by HBM: a pass with both sets moves 6.5 GB in
-// 1.11 ms, 5.8 TB/s, 1.21 times its 10 words per voxel for the rows above and
-// below a wave's.  FP16 on 500 x 468 x 391: 0.87 -> 0.55 ms on the mean; a pass
-// with both sets moves 3.3 GB in 0.61 ms, 5.5 TB/s, but 1.8 times its 10 words,
-// as strips of 4 rows read 6.
+// 1.11 ms, 5.8 TB/s: it reads 1.3 times its 7 words per voxel, for the rows
+// above and below a wave's.  FP16 on 500 x 468 x 391: 0.87 -> 0.55 ms on the
+// mean; a pass with both sets moves 3.3 GB in 0.61 ms, 5.5 TB/s: it reads 2.1
+// times its words (strips of 4 rows, and rows of 1000 bytes, which share lines
+// with their neighbours) and writes 1.2 times.
 constexpr int FGW = 4;                       // waves per workgroup
 
 template <typename S, typename T, typename D, int FIRST, int FGR>

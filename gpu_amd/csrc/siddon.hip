@@ -422,13 +422,10 @@ template <int ES, bool ZQ = false> struct FastWalk {
     // whose alpha has no cancellation left: on nearly level rays, where a plane
     // spans much alpha, the rounding of plane 0's would move every crossing.
     // Returns that plane (restart takes it).
-    __device__ __forceinline__ int rebase_z(const DGeo<float> &d, float s, float c, int col, int row, int src) {
+    __device__ __forceinline__ int rebase_z(const DGeo<float> &d, int row) {
         if (kz == 0.0f) return 0;
-        const float z1 = d.zmin + (float)row * d.dv;
-        float sx, sy, z2;
-        ray_source(d, s, c, d.ymin + (float)col * d.du, z1, src, sx, sy, z2);
         const float n0 = 4.0f * floorf(nfz * 0.25f);
-        bz0 = (fmaf(n0, d.vz, d.bz) - z1) / (z2 - z1);
+        bz0 = (fmaf(n0, d.vz, d.bz) - (d.zmin + (float)row * d.dv)) * d.ivz * kz;
         nfz -= n0;
         az = fmaf(nfz, kz, bz0);
         return (int)n0;
@@ -611,7 +608,7 @@ __global__ __launch_bounds__(256) void k_project_zq(DGeo<float> d, const float *
                 // (16-bit volumes, whose storage rounding hides it and whose
                 // stored updates are dithered from the sums' low bits, do without)
                 int zq = 0;
-                if constexpr (std::is_same<SV, float>::value) zq = fw.rebase_z(d, s, c, col, row, src);
+                if constexpr (std::is_same<SV, float>::value) zq = fw.rebase_z(d, row);
                 const float lo = fw.ac, span = fw.amax - fw.ac;
                 if (p + 1 < S) fw.amax = fmaf(span, (float)(p + 1) / (float)S, lo);
                 if (p > 0) fw.restart(d, fmaf(span, (float)p / (float)S, lo), zq);
