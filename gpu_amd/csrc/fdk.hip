@@ -251,7 +251,13 @@ __device__ __forceinline__ float fdk_weighted(const DGeo<float> &d, const SI *in
     return a * d.dso / sqrtf(x1 * x1 + x2 * x2 + x3 * x3);
 }
 
-template <int LOGN, typename SI, typename SO, bool WEIGHT>
+// DIFF: the transform is longer than the pad and filters the rows' first
+// differences x[n] - x[n-1] (zero outside the row, n = 0 .. R) with the complex
+// spectrum of the taps' running sums (k_ramp_spectrum).  A smooth row's sums of
+// all its pixels, whose rounding the ramp amplifies at high frequencies, then
+// never form: error against FP64 of half ellipses with 1% of noise, 720 columns,
+// 1.1e-7, where the rows themselves give 4.9e-6 and a direct FP32 DFT 2.3e-6.
+template <int LOGN, typename SI, typename SO, bool WEIGHT, bool DIFF>
 __global__ __launch_bounds__(1 << (LOGN - 3)) void k_ramp_sh(const SI *__restrict__ in, SO *__restrict__ out, int R,
                                                             int64_t nrows_total, const float2 *__restrict__ tw,
                                                             const float *__restrict__ H, DGeo<float> d) {
@@ -280,14 +286,29 @@ __global__ __launch_bounds__(1 << (LOGN - 3)) void k_ramp_sh(const SI *__restric
             }
         }
         v[r] = make_float2(a, b);
+        if constexpr (DIFF) buf[lpad(n)] = v[r];
     }
     __syncthreads();
+    if constexpr (DIFF) {
+        // (through LDS; by lane shifts, with the wave ends alone in LDS, the FDK
+        // of 109 views of 271 x 302 takes 297 us, this way 293)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const int n = tid + r * T;
+            if (n > 0 && n <= R) v[r] = csub(v[r], buf[lpad(n - 1)]);
+        }
+    }
     sh_fft<LOGN, false>(v, buf, tid, stw);
-    // H is real and even: filtering a + ib filters both rows
+    // the taps are real: filtering a + ib filters both rows (H itself is also even)
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const float h = H[tid + sh_perm<LOGN>(i) * T];
-        v[i].x *= h; v[i].y *= h;
+        const int k = tid + sh_perm<LOGN>(i) * T;
+        if constexpr (DIFF) {
+            v[i] = twmul<false>(v[i], reinterpret_cast<const float2 *>(H)[k]);
+        } else {
+            const float h = H[k];
+            v[i].x *= h; v[i].y *= h;
+        }
     }
     float2 u[8];
 #pragma unroll
@@ -335,12 +356,16 @@ __global__ __launch_bounds__(256) void k_ramp_tables(RampH rh, int n, float2 *__
 
 // The filter on a transform of n points instead of pad.  A row's R pixels are
 // zero-padded to pad = 2R, so its filtered pixels are the linear convolution
-// with the taps h[m], |m| < R, of the inverse transform of H; any cyclic
-// transform of n >= 2R - 1 points gives the same pixels from the taps'
-// spectrum on n points.  The taps and the spectrum are real and even and are
-// summed in FP64, one wave per value.  A direct DFT of the pad per row pair
-// took 171.4 ms for the FDK of 240 views of 720 x 475 onto 301 x 307 x 187
-// (169 ms of it the filter); this form takes 2.40 ms.
+// with the taps h[m], |m| < R, of the inverse transform of H, and that of the
+// row's first differences with the taps' running sums g[m] = sum h[j], j <= m,
+// -R <= m < R.  Any cyclic transform of n >= 2R points gives the same pixels
+// from the spectrum of g on n points: with T = -h[R] the sum of the taps (all of
+// them, h[R] too, sum to H[0] = 0),
+// (S(k) - T e^(-2 pi i k R / n)) / (1 - e^(-2 pi i k / n)) from the taps' own
+// spectrum S, and R T at k = 0.  The taps and S are real and even and are summed in
+// FP64, one wave per value.  A direct DFT of the pad per row pair took 171.4 ms
+// for the FDK of 240 views of 720 x 475 onto 301 x 307 x 187 (169 ms of it the
+// filter); this form takes 2.45 ms.
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -348,7 +373,7 @@ __device__ __forceinline__ double wave_sum(double v) {
 }
 __global__ __launch_bounds__(256) void k_ramp_taps(RampH rh, int R, double *__restrict__ taps) {
     const int m = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (m >= R) return;
+    if (m > R) return;
     double v = 0.0;
     for (int k = lane; k <= R; k += 64) {   // k and pad - k together (H[0] = 0)
         const int64_t p = (int64_t)k * m % rh.pad;
@@ -358,18 +383,30 @@ __global__ __launch_bounds__(256) void k_ramp_taps(RampH rh, int R, double *__re
     if (lane == 0) taps[m] = v / (double)rh.pad;
 }
 __global__ __launch_bounds__(256) void k_ramp_spectrum(const double *__restrict__ taps, int R, int n,
-                                                       float *__restrict__ H) {
+                                                       float2 *__restrict__ G) {
     const int k = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (k > n / 2) return;
+    // e^(i pi k / n) in lane 0, e^(2 pi i k R / n) in the others
+    double s, c;
+    sincospi(lane == 0 ? (double)k / (double)n : 2.0 * (double)((int64_t)k * R & (n - 1)) / (double)n, &s, &c);
     double v = 0.0;
     for (int m = lane; m < R; m += 64) {
         const int64_t p = (int64_t)k * m & (n - 1);
         v += (m == 0 ? 1.0 : 2.0) * taps[m] * cospi(2.0 * (double)p / (double)n);
     }
     v = wave_sum(v);
+    const double sr = __shfl(s, 1, 64), cr = __shfl(c, 1, 64);
     if (lane != 0) return;
-    H[k] = (float)v;
-    if (k > 0 && k < n / 2) H[n - k] = (float)v;
+    const double t = -taps[R];
+    if (k == 0) {
+        G[0] = make_float2((float)(t * (double)R), 0.0f);
+        return;
+    }
+    // 1 - e^(-iw) = 2 sin(w/2) (sin(w/2) + i cos(w/2))
+    const double qr = v - t * cr, qi = t * sr, f = 0.5 / s;
+    const float gr = (float)((qr * s + qi * c) * f), gi = (float)((qi * s - qr * c) * f);
+    G[k] = make_float2(gr, gi);
+    if (k < n / 2) G[n - k] = make_float2(gr, -gi);
 }
 
 template <typename SI, typename SO>
@@ -379,19 +416,22 @@ template <int LOGN, typename SI, typename SO>
 static void launch_sh(ct_context *ctx, const ct_geometry &g, const void *in, void *out, int64_t rows, int64_t pairs,
                       const float2 *tw, const float *H, bool weighted) {
     const DGeo<float> d = derive<float>(g);
-    if (weighted)
-        hipLaunchKernelGGL((k_ramp_sh<LOGN, SI, SO, true>), dim3((unsigned)pairs), dim3(1 << (LOGN - 3)), 0,
-                           ctx->stream, (const SI *)in, (SO *)out, g.ncols, rows, tw, H, d);
-    else
-        hipLaunchKernelGGL((k_ramp_sh<LOGN, SI, SO, false>), dim3((unsigned)pairs), dim3(1 << (LOGN - 3)), 0,
-                           ctx->stream, (const SI *)in, (SO *)out, g.ncols, rows, tw, H, d);
+    auto go = [&](auto w, auto diff) {
+        hipLaunchKernelGGL((k_ramp_sh<LOGN, SI, SO, decltype(w)::value, decltype(diff)::value>), dim3((unsigned)pairs),
+                           dim3(1 << (LOGN - 3)), 0, ctx->stream, (const SI *)in, (SO *)out, g.ncols, rows, tw, H, d);
+    };
+    using std::true_type;
+    using std::false_type;
+    const bool diff = 2 * g.ncols != 1 << LOGN;
+    if (weighted) diff ? go(true_type(), true_type()) : go(true_type(), false_type());
+    else diff ? go(false_type(), true_type()) : go(false_type(), false_type());
 }
 
 template <typename SI, typename SO>
 static ct_status run_ramp(ct_context *ctx, const ct_geometry &g, const void *in, void *out, int nimg, ct_window window,
                           bool weighted) {
     // rows of up to 2048 pixels: the shortest Stockham transform that holds
-    // the row's linear convolution (2R - 1 points); longer ones: a transform
+    // the row's linear convolution (2R points); longer ones: a transform
     // of the pad itself, if it is a power of two that fits the LDS
     const int R = g.ncols, pad = 2 * R;
     int logn = 9;
@@ -410,11 +450,11 @@ static ct_status run_ramp(ct_context *ctx, const ct_geometry &g, const void *in,
     const int64_t pairs = (rows + 1) / 2;
     if (pairs > 2147483647LL) return fail(ctx, CT_ERR_OVERFLOW, "ramp filter: too many rows");
     ct_status st;
-    char *tab = (char *)slot(ctx, SLOT_FFT, (sizeof(float2) + sizeof(float)) * (size_t)n + sizeof(double) * (size_t)R, &st);
+    char *tab = (char *)slot(ctx, SLOT_FFT, 2 * sizeof(float2) * (size_t)n + sizeof(double) * (size_t)(R + 1), &st);
     if (!tab) return st;
     float2 *dtw = (float2 *)tab;
     double *taps = (double *)(tab + sizeof(float2) * (size_t)n);
-    float *dH = (float *)(taps + R);
+    float *dH = (float *)(taps + R + 1);
     // the frequency step as the reference forms it, in float
     const float du = (float)g.du, dso = (float)g.dso, dod = (float)g.dod;
     const float fmax_ = (float)(1.0 / 2.0 / (double)(du * dso / (dso - dod)));
@@ -422,9 +462,9 @@ static ct_status run_ramp(ct_context *ctx, const ct_geometry &g, const void *in,
     ProfScope ps(ctx, CT_K_RAMP);
     hipLaunchKernelGGL(k_ramp_tables, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, rh, n, dtw, dH);
     if (n != pad) {
-        hipLaunchKernelGGL(k_ramp_taps, dim3((R + 3) / 4), dim3(256), 0, ctx->stream, rh, R, taps);
+        hipLaunchKernelGGL(k_ramp_taps, dim3((R + 4) / 4), dim3(256), 0, ctx->stream, rh, R, taps);
         hipLaunchKernelGGL(k_ramp_spectrum, dim3((n / 2 + 4) / 4), dim3(256), 0, ctx->stream, (const double *)taps, R, n,
-                           dH);
+                           (float2 *)dH);
     }
     switch (logn) {
     case 9: launch_sh<9, SI, SO>(ctx, g, in, out, rows, pairs, dtw, dH, weighted); break;

@@ -851,6 +851,21 @@ def test_ramp_filter_transform_lengths(ctx, ncols):
         assert rel(host(ctx.ramp_filter(g, dev(p), window=window)), ref) <= 1e-5
 
 
+@pytest.mark.parametrize("ncols", [1, 2, 63, 100, 200, 257, 720, 1025, 2047])
+def test_ramp_filter_smooth_rows(ctx, ncols):
+    """Smooth rows, half ellipses with 1% of noise and constant rows, of lengths
+    that are filtered by convolution: within 1e-6 of FP64, some ten roundings of
+    2^-24, where a direct FP32 DFT of the padded row is 1 to 3e-6 off."""
+    g = Geometry(nx=8, ny=8, nz=8, vx=1.0, ncols=ncols, nrows=3, du=0.9, nviews=3, dso=100.0, dod=-50.0)
+    rows = np.sqrt(np.maximum(0.0, 1.0 - np.linspace(-1.1, 1.1, ncols) ** 2)) if ncols > 2 else np.ones(ncols)
+    p = rows + 0.01 * np.random.default_rng(ncols).standard_normal((3, 3, ncols))
+    p[1] = 2.0
+    p = p.astype(np.float32)
+    for window in ("ramp", "hann"):
+        ref = orc.ramp_filter(g, p, window, prec=64)
+        assert rel(host(ctx.ramp_filter(g, dev(p), window=window)), ref) <= 1e-6
+
+
 @pytest.mark.parametrize("ncols", [8, 256, 512, 1024, 2048])
 def test_ramp_filter_power_of_two_pads(ctx, ncols):
     """Pads 2^9..2^12 take the Stockham radix-8 kernel, 16 the radix-2 LDS
